@@ -38,78 +38,105 @@ constexpr int kXcds = 8;        // MI355X accelerator complex dies (one L2 each)
 constexpr int kMaxSteps = 32;   // K steps (4 blocks) per row: K <= 4096
 
 // ---- grouping ---------------------------------------------------------------------------
-// One workgroup: count the (token, slot) entries of every expert, lay the experts out in
-// order (exp_off, tile_off), and give every entry a position inside its expert's range by
-// an LDS counter. The order of the entries inside an expert depends on timing, but nothing
-// computed from them does: each pair's GEMM column and epilogue depend on that pair alone,
-// and a token's pairs are combined in ascending expert order, which the ranges fix.
-__global__ __launch_bounds__(256) void k_group(const int32_t* __restrict__ idx, const float* __restrict__ w,
-                                               int P, int k, int E, int32_t* __restrict__ pair_tok,
-                                               float* __restrict__ pair_w, int32_t* __restrict__ pair_of,
-                                               int32_t* __restrict__ exp_off, int32_t* __restrict__ tile_off) {
+// Count the (token, slot) entries of every expert, lay the experts out in order (exp_off; in
+// tiles of `tile` pairs: tile_off, and each tile's expert) and give every entry a position inside
+// its expert's range by an LDS counter. The order of the entries inside an expert depends on
+// timing, but nothing computed from them does: each pair's GEMM column and epilogue depend on
+// that pair alone, and a token's pairs are combined in ascending expert order, which the ranges
+// fix.
+// A workgroup takes kGroupEntries entries, held in registers between the count and the placement.
+// More entries take several workgroups: k_group_count writes each one's counts, and in k_group
+// every workgroup adds up the counts of those before it (32,768 entries of 128 experts: 103 us
+// in one workgroup of 256 threads that read them twice, 11 us for the two launches).
+constexpr int kGroupJ = 8;  // entries per thread, loaded together
+constexpr int kGroupThreads = 1024;
+constexpr int kGroupEntries = kGroupThreads * kGroupJ;
+
+__device__ __forceinline__ void group_load(const int32_t* __restrict__ idx, int P, int E, int q0, int (&ev)[kGroupJ]) {
+#pragma unroll
+  for (int j = 0; j < kGroupJ; ++j) {
+    const int q = q0 + kGroupThreads * j;
+    ev[j] = q < P ? min(max(idx[q], 0), E - 1) : -1;
+  }
+}
+
+__global__ __launch_bounds__(kGroupThreads) void k_group_count(const int32_t* __restrict__ idx, int P, int E,
+                                                               int32_t* __restrict__ hist) {
   __shared__ int cnt[1024];
-  const int tid = threadIdx.x, lane = tid & 63;
-  for (int e = tid; e < E; e += 256) cnt[e] = 0;
+  const int tid = threadIdx.x;
+  cnt[tid] = 0;
+  int ev[kGroupJ];
+  group_load(idx, P, E, blockIdx.x * kGroupEntries + tid, ev);
   __syncthreads();
-  constexpr int kGJ = 8;  // entries per thread whose loads are issued together (one round trip)
-  const bool one = P <= 256 * kGJ;  // one pass: the entries and weights stay in registers
-  int ev[kGJ];
-  float wv[kGJ];
-  for (int b0 = 0; b0 < P; b0 += 256 * kGJ) {
 #pragma unroll
-    for (int j = 0; j < kGJ; ++j) {
-      const int q = b0 + 256 * j + tid;
-      ev[j] = q < P ? min(max(idx[q], 0), E - 1) : -1;
-      wv[j] = (one && q < P) ? w[q] : 0.f;
-    }
+  for (int j = 0; j < kGroupJ; ++j)
+    if (ev[j] >= 0) atomicAdd(&cnt[ev[j]], 1);
+  __syncthreads();
+  if (tid < E) hist[blockIdx.x * E + tid] = cnt[tid];
+}
+
+__global__ __launch_bounds__(kGroupThreads) void k_group(const int32_t* __restrict__ idx, const float* __restrict__ w,
+                                                         int P, int k, int E, int tile, GroupOut o) {
+  __shared__ int cnt[1024], toff[1025], wsum[2][16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int q0 = blockIdx.x * kGroupEntries + tid;
+  cnt[tid] = 0;
+  int ev[kGroupJ];
+  float wv[kGroupJ];
+  group_load(idx, P, E, q0, ev);
 #pragma unroll
-    for (int j = 0; j < kGJ; ++j)
+  for (int j = 0; j < kGroupJ; ++j) wv[j] = ev[j] >= 0 ? w[q0 + kGroupThreads * j] : 0.f;
+  __syncthreads();
+  int c = 0, before = 0;  // this thread's expert (tid): entries in all, and in earlier workgroups
+  if (gridDim.x == 1) {
+#pragma unroll
+    for (int j = 0; j < kGroupJ; ++j)
       if (ev[j] >= 0) atomicAdd(&cnt[ev[j]], 1);
+    __syncthreads();
+    c = cnt[tid];
+  } else if (tid < E) {
+    for (int b = 0; b < (int)gridDim.x; ++b) {
+      const int v = o.hist[b * E + tid];
+      c += v;
+      before += b < (int)blockIdx.x ? v : 0;
+    }
+  }
+  const int tc = (c + tile - 1) / tile;
+  int po = c, to = tc;  // inclusive prefix over the wave, then over the workgroup, then exclusive
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int a = __shfl_up(po, d, 64), b = __shfl_up(to, d, 64);
+    if (lane >= d) po += a, to += b;
+  }
+  if (lane == 63) wsum[0][wave] = po, wsum[1][wave] = to;
+  __syncthreads();
+  po -= c, to -= tc;
+  for (int v = 0; v < wave; ++v) po += wsum[0][v], to += wsum[1][v];
+  if (tid < E) {
+    cnt[tid] = po + before;  // becomes the next free position
+    toff[tid] = to;
+    if (blockIdx.x == 0) o.exp_off[tid] = po, o.tile_off[tid] = to;
+    if (tid == E - 1) {
+      toff[E] = to + tc;
+      if (blockIdx.x == 0) o.exp_off[E] = po + c, o.tile_off[E] = to + tc;
+    }
   }
   __syncthreads();
-  if (tid < 64) {  // expert offsets, in expert order: lane l takes experts 16l .. 16l+15 (E <= 1024)
-    int c[16], s = 0, ts = 0;
-#pragma unroll
-    for (int u = 0; u < 16; ++u) {
-      const int e = 16 * lane + u;
-      c[u] = e < E ? cnt[e] : 0;
-      s += c[u], ts += (c[u] + kPairTile - 1) / kPairTile;
+  const int n_tiles = toff[E];
+  for (int t = blockIdx.x * kGroupThreads + tid; t < n_tiles; t += gridDim.x * kGroupThreads) {
+    int lo = 0, hi = E;  // toff[lo] <= t < toff[hi]
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (toff[mid] <= t) lo = mid; else hi = mid;
     }
-    int po = s, to = ts;  // inclusive prefix over lanes, then exclusive
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int a = __shfl_up(po, o, 64), b = __shfl_up(to, o, 64);
-      if (lane >= o) po += a, to += b;
-    }
-    po -= s, to -= ts;
-#pragma unroll
-    for (int u = 0; u < 16; ++u) {
-      const int e = 16 * lane + u;
-      if (e < E) {
-        exp_off[e] = po, tile_off[e] = to;
-        cnt[e] = po;  // becomes the next free position
-      }
-      po += c[u], to += (c[u] + kPairTile - 1) / kPairTile;
-    }
-    if (16 * lane < E && E <= 16 * lane + 16) exp_off[E] = po, tile_off[E] = to;
+    o.tile_exp[t] = lo;
   }
-  __syncthreads();
-  for (int b0 = 0; b0 < P; b0 += 256 * kGJ) {
-    if (!one) {
 #pragma unroll
-      for (int j = 0; j < kGJ; ++j) {
-        const int q = b0 + 256 * j + tid;
-        ev[j] = q < P ? min(max(idx[q], 0), E - 1) : -1;
-        wv[j] = q < P ? w[q] : 0.f;
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < kGJ; ++j) {
-      if (ev[j] >= 0) {
-        const int q = b0 + 256 * j + tid;
-        const int pos = atomicAdd(&cnt[ev[j]], 1);
-        pair_tok[pos] = q / k, pair_w[pos] = wv[j], pair_of[q] = pos;
-      }
+  for (int j = 0; j < kGroupJ; ++j) {
+    if (ev[j] >= 0) {
+      const int q = q0 + kGroupThreads * j;
+      const int pos = atomicAdd(&cnt[ev[j]], 1);
+      o.pair_tok[pos] = q / k, o.pair_w[pos] = wv[j], o.pair_of[q] = pos;
     }
   }
 }
@@ -585,7 +612,7 @@ namespace {
 constexpr uint64_t kAlign = 256;
 uint64_t up(uint64_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
 struct GroupedPlan {
-  uint64_t pair_tok, pair_w, pair_of, exp_off, tile_off, img_x, sc_x, img_h, sc_h, obuf;
+  uint64_t pair_tok, pair_w, pair_of, exp_off, tile_off, tile_exp, hist, sc_x, img_h, sc_h, xo;
   uint64_t img_hsh, sc_hsh, osh, sig, total;
 };
 GroupedPlan grouped_plan(uint64_t T, uint64_t k, uint64_t E, uint64_t I, uint64_t H, uint64_t Ish) {
@@ -597,11 +624,14 @@ GroupedPlan grouped_plan(uint64_t T, uint64_t k, uint64_t E, uint64_t I, uint64_
   p.pair_of = o, o += up(P * 4);
   p.exp_off = o, o += up((E + 1) * 4);
   p.tile_off = o, o += up((E + 1) * 4);
-  p.img_x = o, o += up(T * (H / 32) * kImgBytes);
+  p.tile_exp = o, o += up(group_tiles_max(P, E, kGroupTileMin) * 4);
+  p.hist = o, o += up(group_hist_bytes(P, E));
   p.sc_x = o, o += up(T * (H / 32) * 4);
   p.img_h = o, o += up(P * (I / 32) * kImgBytes);
   p.sc_h = o, o += up(P * (I / 32) * 4);
-  p.obuf = o, o += up(P * H * 4);
+  // the x images are last read by the gate/up launches and the down outputs first written by
+  // the down launches: they share xo
+  p.xo = o, o += up(std::max(T * (H / 32) * kImgBytes, P * H * 4));
   p.img_hsh = o, o += up(T * (Ish / 32) * kImgBytes);  // the shared expert (Ish = 0: none)
   p.sc_hsh = o, o += up(T * (Ish / 32) * 4);
   p.osh = o, o += up(Ish ? T * H * 4 : 0);
@@ -625,11 +655,13 @@ GroupedScratch grouped_scratch(const Scratch& s, uint64_t T, uint64_t k, uint64_
   g.pair_of = reinterpret_cast<int32_t*>(b + p.pair_of);
   g.exp_off = reinterpret_cast<int32_t*>(b + p.exp_off);
   g.tile_off = reinterpret_cast<int32_t*>(b + p.tile_off);
-  g.img_x = reinterpret_cast<uint8_t*>(b + p.img_x);
+  g.tile_exp = reinterpret_cast<int32_t*>(b + p.tile_exp);
+  g.hist = reinterpret_cast<int32_t*>(b + p.hist);
+  g.img_x = reinterpret_cast<uint8_t*>(b + p.xo);
   g.sc_x = reinterpret_cast<uint32_t*>(b + p.sc_x);
   g.img_h = reinterpret_cast<uint8_t*>(b + p.img_h);
   g.sc_h = reinterpret_cast<uint32_t*>(b + p.sc_h);
-  g.obuf = reinterpret_cast<float*>(b + p.obuf);
+  g.obuf = reinterpret_cast<float*>(b + p.xo);
   g.img_hsh = reinterpret_cast<uint8_t*>(b + p.img_hsh);
   g.sc_hsh = reinterpret_cast<uint32_t*>(b + p.sc_hsh);
   g.osh = reinterpret_cast<float*>(b + p.osh);
@@ -649,11 +681,20 @@ bool grouped_supported(const mr_layer& L) {
   return true;
 }
 
-hipError_t launch_group(const Launch& K, const int32_t* idx, const float* w, int P, int k, int E, int32_t* pair_tok,
-                        float* pair_w, int32_t* pair_of, int32_t* exp_off, int32_t* tile_off) {
+uint64_t group_hist_bytes(uint64_t P, uint64_t E) {
+  return P > (uint64_t)kGroupEntries ? (P + kGroupEntries - 1) / kGroupEntries * E * 4 : 0;
+}
+
+hipError_t launch_group(const Launch& K, const int32_t* idx, const float* w, int P, int k, int E, int tile,
+                        const GroupOut& o) {
   ProfScope ps(K, "group");
-  hipLaunchKernelGGL(k_group, dim3(1), dim3(256), 0, K.s, idx, w, P, k, E, pair_tok, pair_w, pair_of, exp_off,
-                     tile_off);
+  const dim3 grid((unsigned)((P + kGroupEntries - 1) / kGroupEntries));
+  if (grid.x > 1) {
+    hipLaunchKernelGGL(k_group_count, grid, dim3(kGroupThreads), 0, K.s, idx, P, E, o.hist);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL(k_group, grid, dim3(kGroupThreads), 0, K.s, idx, w, P, k, E, tile, o);
   return hipGetLastError();
 }
 
@@ -685,9 +726,8 @@ hipError_t launch_grouped(const Launch& K, const mr_layer& L, const float* x, ui
   const int P = (int)T * k;
   const int max_tiles = (P + kPairTile - 1) / kPairTile + E;
   hipError_t e;
-  if ((e = launch_group(K, idx, w, P, k, E, gs.pair_tok, gs.pair_w, gs.pair_of, gs.exp_off, gs.tile_off)) !=
-      hipSuccess)
-    return e;
+  const GroupOut go{gs.pair_tok, gs.pair_w, gs.pair_of, gs.exp_off, gs.tile_off, gs.tile_exp, gs.hist};
+  if ((e = launch_group(K, idx, w, P, k, E, kPairTile, go)) != hipSuccess) return e;
   {
     ProfScope ps(K, "split_x");
     hipLaunchKernelGGL(k_split_rows, dim3((unsigned)((H / 32 + 31) / 32), std::min<uint32_t>(T, 65535u)), dim3(256), 0,
@@ -708,6 +748,25 @@ hipError_t launch_grouped(const Launch& K, const mr_layer& L, const float* x, ui
                        K.s, a);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
+  // The shared expert (layer.rs:1898-1953): one group of every token on the same x images,
+  // weight 1 and SiLU (the routed experts' activation does not apply), its down outputs
+  // [T][H], then sigmoid(x . gate_inp) per token, which the combine applies after the routed
+  // sum.
+  const int Ish = L.d.sh_gate ? (int)L.Ish : 0, tiles = ((int)T + kPairTile - 1) / kPairTile;
+  if (Ish) {
+    GroupedArgs sg{};
+    sg.w0 = expert_loc(L.d.sh_gate), sg.w1 = expert_loc(L.d.sh_up);
+    sg.img = gs.img_x, sg.isc = gs.sc_x, sg.single_p = (int)T;
+    sg.himg = gs.img_hsh, sg.hsc = gs.sc_hsh;
+    sg.M = Ish, sg.K = H, sg.E = 1, sg.act = MR_ACT_SILU;
+    {
+      ProfScope ps(K, "grouped_shared_gateup");
+      constexpr int rows = kRowsOf<true>;
+      hipLaunchKernelGGL(k_grouped_gemm<true>, dim3(grouped_grid((uint64_t)((Ish + rows - 1) / rows) * tiles)),
+                         dim3(kGW * 64), 0, K.s, sg);
+      if ((e = hipGetLastError()) != hipSuccess) return e;
+    }
+  }
   GroupedArgs d{};
   d.w0 = expert_loc(L.d.down);
   d.img = gs.img_h, d.isc = gs.sc_h, d.pair_tok = nullptr, d.pair_w = gs.pair_w;
@@ -720,24 +779,7 @@ hipError_t launch_grouped(const Launch& K, const mr_layer& L, const float* x, ui
                        K.s, d);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
-  if (!L.d.sh_gate) return launch_combine(K, gs.obuf, gs.pair_of, idx, w, L.d.down_bias, T, k, H, nullptr, nullptr, y);
-  // The shared expert (layer.rs:1898-1953): one group of every token on the same x images,
-  // weight 1 and SiLU (the routed experts' activation does not apply), its down outputs
-  // [T][H], then sigmoid(x . gate_inp) per token, which the combine applies after the routed
-  // sum.
-  const int Ish = (int)L.Ish, tiles = ((int)T + kPairTile - 1) / kPairTile;
-  GroupedArgs sg{};
-  sg.w0 = expert_loc(L.d.sh_gate), sg.w1 = expert_loc(L.d.sh_up);
-  sg.img = gs.img_x, sg.isc = gs.sc_x, sg.single_p = (int)T;
-  sg.himg = gs.img_hsh, sg.hsc = gs.sc_hsh;
-  sg.M = Ish, sg.K = H, sg.E = 1, sg.act = MR_ACT_SILU;
-  {
-    ProfScope ps(K, "grouped_shared_gateup");
-    constexpr int rows = kRowsOf<true>;
-    hipLaunchKernelGGL(k_grouped_gemm<true>, dim3(grouped_grid((uint64_t)((Ish + rows - 1) / rows) * tiles)),
-                       dim3(kGW * 64), 0, K.s, sg);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-  }
+  if (!Ish) return launch_combine(K, gs.obuf, gs.pair_of, idx, w, L.d.down_bias, T, k, H, nullptr, nullptr, y);
   GroupedArgs sd{};
   sd.w0 = expert_loc(L.d.sh_down);
   sd.img = gs.img_hsh, sd.isc = gs.sc_hsh, sd.single_p = (int)T, sd.out = gs.osh;

@@ -1,78 +1,135 @@
 // mr_grouped_q4k.hip -- multi-token (prefill / batched) Q4_K MoE experts as grouped GEMMs on
-// the gfx950 int8 MFMA (v_mfma_i32_16x16x32_i8).
+// the gfx950 f16 MFMA (v_mfma_f32_16x16x32_f16).
 //
 // The reference runs each expert once over all of its tokens (index_select, gate/up/act/down,
 // index_add: layer.rs:2148-2183; on the GPU one projection per expert, metal/mod.rs:911-962).
 // Here, after the grouping of mr_grouped.hip (k_group: (token, slot) pairs by expert):
-//   k_split_q4k        activation rows -> two int8 terms per element and a scale per 256-element
-//                      super-block: v = s*(t0 + t1/128), s = max|v|/127 (|error| <= s/256), plus
-//                      the f32 sum of every 32-element sub-block.
-//   k_grouped_q4k<1>   gate and up for one (expert, 32-row tile, 32-pair tile); epilogue bias +
-//                      activation x routing weight -> h [pair][I] (f32).
-//   k_split_q4k        h rows -> terms.
-//   k_grouped_q4k<0>   down for one (expert, 64-row tile, 32-pair tile) -> o [pair][H].
+//   k_split_f16        activation rows -> two f16 terms per element (the f16 nearest to x * p and
+//                      the f16 nearest to the rest, p a power of two per row: 22 significant
+//                      bits) plus the f32 sum of every 32-element sub-block as three f16 terms;
+//                      with a shared expert also its sigmoid gate of the row.
+//   k_grouped_q4k<1>   gate and up for one (expert, 256 rows, pair tile); epilogue bias +
+//                      activation x routing weight, split into the down input images (a tile's
+//                      256 rows are one super-block of the down input, with its own p).
+//   k_grouped_q4k<0>   down for one (expert, 256 rows, pair tile) -> o [pair][H].
 //   k_combine          (mr_grouped.hip) the pairs of a token in ascending expert order, then the
 //                      shared expert scaled by its sigmoid gate (layer.rs:1092-1106, 1935-1951).
-// A work item reads its expert's weight rows once for its 32 pairs, so an expert's weights are
-// read ceil(n_e / 32) times per call (from HBM once, the repeats from the XCD's L2), against once
-// per (token, slot) on the per-token path.
+// The shared expert is one more group (every token, weight 1, SiLU) of the same two launches.
 //
-// Arithmetic per sub-block j of a Q4_K super-block (dequant.rs:218-262 regrouped):
-//   sum_k w_k x_k = d*sc_j * sum_k q_k x_k - (dmin*m_j) * sum_k x_k,
-// with sum_k q_k x_k = s * (A0 + A1/128), A_t = sum_k q_k t_k exact in int32 (one MFMA per term:
-// A = 16 rows x 32 nibbles as int8, B = 32 elements x 16 pairs). The sc_j weighting is summed
-// over the super-block in int32 (|sum| < 8 * 63 * 32*15*127 < 2^31), then scaled by d*s in f32.
+// Arithmetic per 256-element super-block (dequant.rs:218-262 regrouped):
+//   sum_k w_k x_k = d * sum_k (sc_j q_k) x_k - dmin * sum_j m_j X_j,
+// with sc_j q_k <= 63 * 15 = 945 an exact f16, so the first sum is one f16 MFMA chain per term
+// over all eight sub-blocks (products of 10 by 11 bits, f32 accumulation) and needs no work on
+// its accumulators per sub-block; the second is one MFMA (m_j exact, X_j in three f16 terms).
 #include "mr_device.h"
 #include "mr_fused_common.h"
 #include "mr_internal.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace mr {
 
-typedef int i32x4v __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
-constexpr int kQPairs = 32;    // pairs per work item (2 MFMA column groups of 16)
 constexpr int kQXcds = 8;      // workgroups are dispatched round robin over the 8 XCDs
+// Image of one (row, super-block): 8 K steps n = 4h + 2u + hl, each [term][lane group g][8 halves],
+// then the sub-block sums [term 0..2, zero][8 halves]. Half j of (n, g) is element
+// 128 h + 64 (g / 2) + 32 hl + 16 (g % 2) + 8 u + kQPerm[j]: a weight lane of group g holds 16 of
+// the 64 quant bytes of half h (low nibbles of one sub-block, hl = 0, high nibbles of the next),
+// takes 8 of them per u, and unpacks bytes 0, 2 and 1, 3 of a dword into two pairs of halves.
+constexpr int kQImgSb = 8 * 128 + 64;
+// Offset past every buffer of the GEMM (images: at most this many bytes, weight matrices: far
+// fewer): a load there fetches nothing and reads zero.
+constexpr int kPast = 0x7F000000;
+__device__ constexpr int kQPerm[8] = {0, 2, 1, 3, 4, 6, 5, 7};  // its own inverse
 
-// ---- activation rows -> terms ---------------------------------------------------------------
-// One wave per (row, 256-element super-block): lane l holds elements 4l .. 4l+3.
-__global__ __launch_bounds__(256) void k_split_q4k(const float* __restrict__ src, int n_rows, int D,
-                                                   int8_t* __restrict__ t0, int8_t* __restrict__ t1,
-                                                   float* __restrict__ s_out, float* __restrict__ x_sum) {
-  const int lane = threadIdx.x & 63;
-  const int nsb = D >> 8;
-  const int64_t item = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (item >= (int64_t)n_rows * nsb) return;  // uniform per wave
-  const int64_t r = item / nsb;
-  const int sb = (int)(item - r * nsb);
-  const size_t off = (size_t)r * D + (size_t)sb * 256 + 4 * lane;
-  const f32x4 v = *reinterpret_cast<const f32x4*>(src + off);
-  float mx = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
-  mx = wave_max(mx);
-  // sub-block sums: lanes 8j .. 8j+7 hold sub-block j (elements in order within a lane, then
-  // a butterfly over the 8 lanes)
-  float ps = (v.x + v.y) + (v.z + v.w);
-  ps += __shfl_xor(ps, 1, 64);
-  ps += __shfl_xor(ps, 2, 64);
-  ps += __shfl_xor(ps, 4, 64);
-  const float s = mx / 127.f;
-  const float inv = mx > 0.f ? 127.f / mx : 0.f;
-  const float inv1 = mx > 0.f ? 128.f * inv : 0.f;
-  uint32_t w0 = 0, w1 = 0;
+__device__ __forceinline__ uint32_t f16_bits(float v) { return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)v); }
+// v = hi + lo, the two terms of the split (each rounded to nearest)
+__device__ __forceinline__ void split2(float v, uint32_t& hi, uint32_t& lo) {
+  const _Float16 h = (_Float16)v;
+  hi = (uint32_t)__builtin_bit_cast(uint16_t, h);
+  lo = f16_bits(v - (float)h);
+}
+// The power of two p that brings a largest magnitude mx to [2^14, 2^15) (mx = 0: 1), and 1/p.
+__device__ __forceinline__ void pow2_scale(float mx, float& p, float& pinv) {
+  const int ex = (int)((__float_as_uint(mx) >> 23) & 0xFFu);  // biased; 0: zero or denormal
+  const int pe = mx > 0.f ? min(max(127 + 14 + 127 - ex, 2), 252) : 127;
+  p = __uint_as_float((uint32_t)pe << 23);
+  pinv = __uint_as_float((uint32_t)(254 - pe) << 23);
+}
+// Sub-block sum X (already scaled by p) -> its three f16 terms of 2^-5 X (32 elements below
+// 2^15 sum to less than 2^20, past f16).
+__device__ __forceinline__ uint32_t sum_term(float X, int t) {
+  float r = X * 0.03125f;
+  uint32_t b = 0u;
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const float x = v[c];
-    const float a = fminf(fmaxf(rintf(x * inv), -127.f), 127.f);
-    const float res = __builtin_fmaf(-a, s, x);  // x - s*t0, one rounding
-    const float b = fminf(fmaxf(rintf(res * inv1), -127.f), 127.f);
-    w0 |= ((uint32_t)(int)a & 0xFFu) << (8 * c);
-    w1 |= ((uint32_t)(int)b & 0xFFu) << (8 * c);
+  for (int q = 0; q < 3; ++q) {
+    const _Float16 h = (_Float16)r;
+    if (q == t) b = (uint32_t)__builtin_bit_cast(uint16_t, h);
+    r = r - (float)h;
   }
-  *reinterpret_cast<uint32_t*>(t0 + off) = w0;
-  *reinterpret_cast<uint32_t*>(t1 + off) = w1;
-  if (lane == 0) s_out[(size_t)r * nsb + sb] = s;
-  if ((lane & 7) == 0) x_sum[(size_t)r * (D >> 5) + sb * 8 + (lane >> 3)] = ps;
+  return b;
+}
+
+// Bounds-checked buffer of nbytes (raw, 32-bit offsets).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const uint8_t* p, uint32_t nbytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p), 0, (int)nbytes, 0x00027000);
+}
+
+// ---- activation rows -> images ----------------------------------------------------------------
+// One workgroup per row, its waves over the row's super-blocks in turn (lane l: elements 4l ..
+// 4l+3), twice: the row's largest magnitude, then the split (the second read hits L1). sig: the
+// shared expert's gate sigmoid(x . gate_inp) of the row, 1 without gate_inp (layer.rs:1935-1951).
+__global__ __launch_bounds__(256) void k_split_f16(const float* __restrict__ src, int D, uint8_t* __restrict__ img,
+                                                   float* __restrict__ pinv_out, const float* __restrict__ gi,
+                                                   float* __restrict__ sig) {
+  __shared__ float red[8];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int nsb = D >> 8;
+  const int64_t r = blockIdx.x;
+  const float* row = src + (size_t)r * D;
+  float mx = 0.f, z = 0.f;
+  for (int sb = wave; sb < nsb; sb += 4) {
+    const f32x4 v = *reinterpret_cast<const f32x4*>(row + sb * 256 + 4 * lane);
+    mx = fmaxf(mx, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+    if (gi) {
+      const f32x4 gv = *reinterpret_cast<const f32x4*>(gi + sb * 256 + 4 * lane);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) z = __builtin_fmaf(v[c], gv[c], z);
+    }
+  }
+  mx = wave_max(mx);
+  if (gi) z = wave_sum_fast(z);
+  if (lane == 0) red[wave] = mx, red[4 + wave] = z;
+  __syncthreads();
+  mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  float p, pinv;
+  pow2_scale(mx, p, pinv);
+  if (threadIdx.x == 0) {
+    pinv_out[r] = pinv;
+    if (sig) sig[r] = gi ? sigmoidf_((red[4] + red[5]) + (red[6] + red[7])) : 1.0f;
+  }
+  // element 4l + c of the super-block: h = l >> 5, g / 2 = l >> 4 & 1, hl = l >> 3 & 1, g % 2 =
+  // l >> 2 & 1, u = l >> 1 & 1, bytes 4 (l & 1) + c, i.e. halves 4 (l & 1) + {0, 2, 1, 3}
+  const int at = (4 * (lane >> 5) + (lane & 2) + ((lane >> 3) & 1)) * 128 +
+                 (2 * ((lane >> 4) & 1) + ((lane >> 2) & 1)) * 16 + (lane & 1) * 8;
+  for (int sb = wave; sb < nsb; sb += 4) {
+    const f32x4 v = *reinterpret_cast<const f32x4*>(row + sb * 256 + 4 * lane);
+    uint8_t* dst = img + ((size_t)r * nsb + sb) * kQImgSb;
+    uint32_t h[4], l[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) split2(v[c] * p, h[c], l[c]);
+    *reinterpret_cast<uint2*>(dst + at) = make_uint2(h[0] | h[2] << 16, h[1] | h[3] << 16);
+    *reinterpret_cast<uint2*>(dst + at + 64) = make_uint2(l[0] | l[2] << 16, l[1] | l[3] << 16);
+    float ps = (v.x + v.y) + (v.z + v.w);  // sub-block sum over the 8 lanes 8j .. 8j+7
+    ps += dpp_f<kDppXor1>(ps);
+    ps += dpp_f<kDppXor2>(ps);
+    ps = add_xor4(ps);
+    const int t = lane & 7, j = lane >> 3;
+    if (t < 4) *reinterpret_cast<uint16_t*>(dst + 1024 + t * 16 + kQPerm[j] * 2) = (uint16_t)sum_term(ps * p, t);
+  }
 }
 
 // ---- shared-expert gate: sigmoid(x . gate_inp) per token (layer.rs:1935-1951) -------------------
@@ -89,272 +146,431 @@ __global__ __launch_bounds__(64) void k_sh_gate(const float* __restrict__ x, int
 }
 
 // ---- grouped GEMM ---------------------------------------------------------------------------
+struct GQ4Group {
+  ExpertLoc w0;        // gate (GATEUP) or down
+  ExpertLoc w1;        // up (GATEUP)
+  const float* b0;     // gate bias [E][M] or null (GATEUP)
+  const float* b1;     // up bias
+  const uint8_t* img;  // images [rows][K/256]
+  const float* pinv;   // their 1/p: [rows] (GATEUP), [rows][K/256] (down)
+  uint8_t* himg;       // GATEUP: the down input images [pairs][M/256]
+  float* hpinv;        // and their 1/p
+  float* out;          // down: [pairs][M]
+  int M, K, act;
+};
 struct GQ4Args {
-  ExpertLoc w0;              // gate (GATEUP) or down
-  ExpertLoc w1;              // up (GATEUP)
-  const float* b0;           // gate bias [E][M] or null (GATEUP)
-  const float* b1;           // up bias
-  const int8_t* t0;          // B terms [rows][K]
-  const int8_t* t1;
-  const float* bs;           // [rows][K/256] term scale
-  const float* bx;           // [rows][K/32] sub-block sums
-  const int32_t* pair_tok;   // B row of pair p, or null (row = p)
-  const float* pair_w;       // GATEUP: routing weight of pair p, or null (1)
-  const int32_t* exp_off;    // [E+1] pair offsets (null: one expert of single_p pairs)
-  const int32_t* tile_off;   // [E+1] 32-pair tile offsets
-  int single_p;
-  float* out;                // GATEUP: h [P][M]; down: o [P][M]
-  int M, K, E, act;
+  GQ4Group r, s;             // routed experts; the shared expert over tokens 0 .. sh_T - 1
+  const int32_t* pair_tok;   // GATEUP: image row of pair p (down: row = p)
+  const float* pair_w;       // GATEUP: routing weight of pair p
+  const int32_t* exp_off;    // [E+1] pair offsets
+  const int32_t* tile_off;   // [E+1] pair tile offsets
+  const int32_t* tile_exp;   // expert of each pair tile
+  int E, sh_T;               // sh_T = 0: no shared expert
   float alpha, limit;
 };
 
-// Work item: (expert e, row tile, 32-pair tile); 4 waves of 16 rows each (gate/up: waves 0-1 gate,
-// 2-3 up, the same 32 rows; down: 64 rows). Per 256-element super-block of K:
-//   A: the wave's 16 rows x 144 bytes as 16-byte pieces (3 loads per lane, each covering about
-//      seven rows' whole super-blocks), one super-block ahead in registers, then written to the
-//      wave's LDS slice; lanes g = 0 decode their row's 16-byte header from it (d, dmin*m_j, sc_j)
-//      and lane (i, g) reads the 8 bytes of row i that hold elements [8g, 8g+8) of a sub-block
-//      pair (low nibbles: even sub-blocks, high: odd).
-//   B: the pairs' two term rows (32 x 2 x 256 bytes), scales and sub-block sums, staged in LDS by
-//      all 256 threads (one super-block ahead in registers, double-buffered LDS) in MFMA operand
-//      order: the 8 bytes that lane l takes for (term, pair group, sub-block j) sit in slot
-//      l ^ 2j of a 512-byte block, so every LDS read of a wave is 64 consecutive 8-byte slots
-//      and the staging writes of one pair's 16 chunks spread over 8 bank pairs.
-//   min term: sum_j (dmin*m_j)[row] * X_j[pair] is a [16 x 8] x [8 x 16] f32 product per pair
-//      group, two v_mfma_f32_16x16x4_f32 per super-block instead of 8 FMAs per lane and sub-block.
-// D layout of the MFMAs: lane (i, g) holds rows 4g .. 4g+3 of the wave's tile, pair column i.
-template <bool GATEUP>
-__global__ __launch_bounds__(256, 3) void k_grouped_q4k(GQ4Args a) {
-  __shared__ __align__(16) uint8_t bst[2][2 * 2 * 8 * 512];  // [buf][term][pair group][sub-block][64 slots x 8 B]
-  __shared__ float bsx[2][2 * 2 * 64];                       // [buf][pair group][j / 4][lane]: sub-block sums
-  __shared__ float bss[2][kQPairs];                          // term scales
-  __shared__ __align__(16) int hsc[4][8][16];                // [wave][sub-block][row] sc_j
-  __shared__ float hm[4][2 * 64];                            // [wave][j / 4][lane]: dmin*m_j of row lane & 15
-  __shared__ __align__(16) float hd[4][16];                  // d
-  __shared__ __align__(16) uint8_t ast[4][16 * 144];         // [wave][row][super-block bytes]
-  __shared__ float pw[kQPairs];                                    // routing weights (GATEUP)
+// Work item: (expert e, 256 rows of each matrix, tile of 16 PG pairs). Gate/up: 16 waves, wave w
+// rows 16 w .. 16 w + 15 of the gate and of the up matrix, so that a lane holds both values of a
+// (row, pair) and a down input super-block (256 rows of h) forms inside one item; down: 8 waves of
+// 32 rows (PG = 1: two workgroups on a CU) or 4 of 64 rows (PG = 4: 323 instead of 348 us at the
+// size below, as its accumulators fit there). The activations are the MFMA's A operand (rows:
+// pairs), the weights its B operand (columns: weight rows): lane (i, g) = lane % 16, lane / 16
+// holds weight row i of every tile, and of D weight row i for pairs 4g .. 4g+3 of each pair group.
+//   A wave's weights come in halves of a super-block, 64 bytes per row, one or two halves ahead in
+//   registers; four lanes load a row's 64 bytes (16 rows per load), and an LDS slice of the wave
+//   turns them into operand order. Lane (i, g) unpacks a nibble pair of row i with one and (two
+//   f16 denormals q 2^-24 or 16 q 2^-24) and one packed multiply by sc 2^10 or sc 2^6, which is
+//   exact: sc q 2^-14.
+//   Images are staged in LDS in operand order (1 KB per (K step, term, pair group)), kKS K steps
+//   per stage, double buffered, one stage ahead in registers, loaded like the weights, four
+//   lanes per row. In both the 16-byte pieces of a row are spread over the banks (xor).
+//   Nothing in the loop may spill: a reload's wait would drain the prefetched loads (measured:
+//   PG = 1 gate/up 90 us with 36 registers spilled, 50 us with none).
+// What bounds it: MFMA and VALU issue, which this chip hardly overlaps (measured on two waves of a
+// SIMD: an MFMA of 16.7 cycles plus four VALU of 2.7 take 26.3), at a clock that falls to 1.7 GHz
+// on long batches: 128 experts of 768 x 2048, 32,768 pairs: gate/up 1.00 -> 0.60 ms and down
+// 0.49 -> 0.32 ms against the int8 MFMA with its scale products on the accumulators per sub-block.
+// Few pairs: the same unpacking against the weight stream (512 experts of 512 x 2048, 3,840
+// pairs: gate/up 300 -> 225 us, 2.7 TB/s; 128 pairs of 128 experts of 768 x 2048: 78 -> 48 us).
+// 16-row tiles per wave (see the kernel), and its waves
+constexpr int q4_tiles(bool gateup, int pg) { return gateup || pg == 1 ? 2 : 4; }
+constexpr int q4_waves(bool gateup, int pg) { return (gateup ? 32 : 16) / q4_tiles(gateup, pg); }
+
+template <bool GATEUP, int PG>
+__global__ __launch_bounds__(64 * q4_waves(GATEUP, PG), q4_tiles(GATEUP, PG) == 4 ? 2 : 4) void k_grouped_q4k(GQ4Args a) {
+  constexpr int NT = q4_tiles(GATEUP, PG), NW = q4_waves(GATEUP, PG);
+  constexpr int kTM = GATEUP ? NT / 2 : NT;  // tiles of one matrix per wave
+  constexpr int kPF = PG == 1 ? 2 : 1;       // half super-blocks of weights in flight
+  constexpr int kKS = PG == 1 ? 8 : 2;       // K steps per stage
+  constexpr int kNS = 8 / kKS;               // stages per super-block
+  constexpr int kPW = kKS * 2 * PG / NW;     // stage pieces (K step, term, pair group) per wave
+  constexpr int kStage = kKS * 2 * PG * 1024;
+  constexpr int kPairs = 16 * PG;
+  constexpr int kEpRow = kQImgSb + 16;  // epilogue: bytes between the images of two pairs
+  constexpr int kEp = GATEUP ? kPairs * kEpRow : 0;
+  __shared__ __align__(16) uint8_t lds[kEp > 2 * kStage ? kEp : 2 * kStage];
+  __shared__ __align__(16) uint8_t xst[2][PG == 1 ? 16 : PG * 1024];  // sub-block sums, operand order (PG = 1: in registers)
+  __shared__ __align__(16) uint8_t ast[NW][NT * 1024];  // half a super-block of the wave's rows: [tile][row][64 bytes]
+  __shared__ __align__(16) uint8_t hst[NW][NT * 256];   // and their headers: [tile][row][16 bytes]
+  __shared__ __align__(16) float pst[2][kPairs];       // down: 1/p of (pair, super-block); gate/up: [0] of the pair
+  __shared__ __align__(16) float pw[kPairs];           // GATEUP: routing weights
+  __shared__ __align__(16) float wred[GATEUP ? NW : 1][kPairs], wsum[GATEUP && NT == 2 ? NW : 1][kPairs];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int i = lane & 15, g = lane >> 4;
-  constexpr int kRows = GATEUP ? 32 : 64;  // output rows of one matrix per work item
-  const int n_rt = (a.M + kRows - 1) / kRows;
-  const int n_tiles = a.exp_off ? a.tile_off[a.E] : (a.single_p + kQPairs - 1) / kQPairs;
-  const int n_work = n_rt * n_tiles;
+  const int n_sh_t = (a.sh_T + kPairs - 1) / kPairs;
+  const int n_rt_s = (a.s.M + 255) >> 8, n_rt_r = (a.r.M + 255) >> 8;
+  const int n_sh = a.sh_T ? n_rt_s * n_sh_t : 0;
+  const int n_work = n_sh + n_rt_r * a.tile_off[a.E];
   const int per_xcd = (n_work + kQXcds - 1) / kQXcds;
   const int loc = blockIdx.x / kQXcds;
-  const int w = (blockIdx.x % kQXcds) * per_xcd + loc;
+  int w = (blockIdx.x % kQXcds) * per_xcd + loc;
   if (loc >= per_xcd || w >= n_work) return;  // uniform
-  int e = 0, tl = 0, rt = 0, p0 = 0, np = 0;
-  if (a.exp_off) {
-    int lo = 0, hi = a.E;  // expert: n_rt * tile_off[e] <= w < n_rt * tile_off[e+1]
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (n_rt * a.tile_off[mid] <= w) lo = mid; else hi = mid;
-    }
-    e = lo;
-    const int nt_e = a.tile_off[e + 1] - a.tile_off[e];
-    const int wl = w - n_rt * a.tile_off[e];
-    rt = wl / nt_e, tl = wl - rt * nt_e;
-    p0 = a.exp_off[e] + tl * kQPairs;
-    np = min(kQPairs, a.exp_off[e + 1] - p0);
+  const bool sh = w < n_sh;
+  const GQ4Group& q = sh ? a.s : a.r;
+  int e = 0, rt, p0, np;
+  if (sh) {
+    rt = w / n_sh_t;
+    p0 = (w - rt * n_sh_t) * kPairs;
+    np = min(kPairs, a.sh_T - p0);
   } else {
-    rt = w / n_tiles, tl = w - rt * n_tiles;
-    p0 = tl * kQPairs;
-    np = min(kQPairs, a.single_p - p0);
+    w -= n_sh;
+    e = a.tile_exp[w / n_rt_r];  // items n_rt tile_off[e] .. n_rt tile_off[e+1] - 1 are expert e's
+    const int t_beg = a.tile_off[e], nt_e = a.tile_off[e + 1] - t_beg, wl = w - n_rt_r * t_beg;
+    rt = wl / nt_e;
+    p0 = a.exp_off[e] + (wl - rt * nt_e) * kPairs;
+    np = min(kPairs, a.exp_off[e + 1] - p0);
   }
-  const int nsb = a.K >> 8;
-  const uint64_t rb = (uint64_t)nsb * 144;
-  const int m = GATEUP ? (wave >> 1) : 0;
-  const int wrow0 = rt * kRows + (GATEUP ? (wave & 1) : wave) * 16;
-  const bool tile_in = wrow0 < a.M;  // uniform
-  const uint8_t* W = expert_at(m ? a.w1 : a.w0, e);
-  // A pieces of this lane: slot it*64 + lane < 144 = (row slot / 9, 16-byte piece slot % 9)
-  const uint8_t* asrc[3];
-  int adst[3];
+  const int M = q.M, nsb = q.K >> 8;
+  const uint32_t rb = (uint32_t)nsb * 144u;
+  // tile t of this wave: GATEUP: gate (t < kTM) or up rows wrow0 + 16 (t % kTM) .. ; down: rows wrow0
+  // + 16 t .. . M % 256 == 0.
+  const int wrow0 = rt * 256 + wave * (16 * kTM);
+  // Buffer loads: one lane offset for all tiles, the tile and super-block in the scalar offset.
+  const __amdgpu_buffer_rsrc_t wb0 = buffer_of(expert_at(q.w0, e), (uint32_t)M * rb);
+  const __amdgpu_buffer_rsrc_t wb1 = GATEUP ? buffer_of(expert_at(q.w1, e), (uint32_t)M * rb) : wb0;
+  uint32_t wt[NT];  // uniform
 #pragma unroll
-  for (int it = 0; it < 3; ++it) {
-    const int sl = min(it * 64 + lane, 143);
-    asrc[it] = W + (uint64_t)min(wrow0 + sl / 9, a.M - 1) * rb + (sl % 9) * 16;
-    adst[it] = (sl / 9) * 144 + (sl % 9) * 16;
-  }
-  if (GATEUP && tid < kQPairs) pw[tid] = a.pair_w ? a.pair_w[p0 + min(tid, np - 1)] : 1.f;
+  for (int t = 0; t < NT; ++t) wt[t] = (uint32_t)(wrow0 + 16 * (t % kTM)) * rb;
+  // loads take 4 lanes per row: row lr, 16-byte piece lp; headers one lane per row
+  const int lr = lane >> 2, lp = lane & 3;
+  const int aoff = lr * (int)rb + 16 + 16 * lp;
+  // header of tile g % NT, row i
+  const uint8_t* hsrc = expert_at(GATEUP && g % NT >= kTM ? q.w1 : q.w0, e) + (uint32_t)(wrow0 + 16 * (g % kTM) + i) * (uint64_t)rb;
+  const int awr = (lr * 4 + (lp ^ (lr >> 2))) * 16, ard = (i * 4 + (g ^ (i >> 2))) * 16;  // in a tile of ast
+  const int bwr = (lp * 16 + (lr ^ (4 * lp))) * 16, brd = (g * 16 + (i ^ (4 * g))) * 16;  // in a stage piece
+  const int32_t* tok = GATEUP && !sh ? a.pair_tok : nullptr;
 
-  // B pieces of this thread: piece j*256 + tid = (term, pair, 16-byte chunk); the chunk holds
-  // elements [8 g0, 8 g0 + 16) of sub-block ch / 2, g0 = 2 (ch & 1): two operand slots
-  const int8_t* bsrc[4];
-  int bdst0[4], bdst1[4];
+  auto run = [&](auto npg_c) {
+    constexpr int NPG = decltype(npg_c)::value;  // pair groups of this item that hold pairs
+    // Stage pieces of this thread: pieces wave kPW .. + kPW - 1, piece (K step, term, pair group) in
+    // that order; 4 lanes bring the 64 bytes of pair 16 pg + lr. Buffer loads
+    // from the images of this call's rows (GATEUP; at most kPast bytes) or of the item's pairs.
+    const uint32_t ib = (uint32_t)nsb * kQImgSb;
+    const __amdgpu_buffer_rsrc_t xb = buffer_of(GATEUP ? q.img : q.img + (size_t)p0 * ib, kPast);
+    auto row_of = [&](int pl) {  // image row of pair pl of the item
+      const int pc = min(pl, np - 1);
+      return GATEUP ? (tok ? tok[p0 + pc] : p0 + pc) : pc;
+    };
+    uint32_t brow[kPW];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int pc = j * 256 + tid;
-    const int term = pc >> 9, pr = (pc >> 4) & 31, ch = pc & 15;
-    const int p = p0 + min(pr, np - 1);
-    const int row = a.pair_tok ? a.pair_tok[p] : p;
-    bsrc[j] = (term ? a.t1 : a.t0) + (size_t)row * a.K + ch * 16;
-    const int sbj = ch >> 1, g0 = 2 * (ch & 1), ii = pr & 15;
-    const int blk = ((term * 2 + (pr >> 4)) * 8 + sbj) * 512;
-    bdst0[j] = blk + ((16 * g0 + ii) ^ (2 * sbj)) * 8;
-    bdst1[j] = blk + ((16 * (g0 + 1) + ii) ^ (2 * sbj)) * 8;
-  }
-  // this thread's sub-block sum (pair tid / 8, sub-block tid % 8) in B operand order
-  const int xdst = (((tid >> 3) >> 4) * 2 + ((tid & 7) >> 2)) * 64 + 16 * (tid & 3) + ((tid >> 3) & 15);
-  const int xrow = [&] {  // pair of this thread's sub-block sum (tid = pair * 8 + sub-block)
-    const int p = p0 + min(tid >> 3, np - 1);
-    return a.pair_tok ? a.pair_tok[p] : p;
-  }();
-  const int srow = [&] {
-    const int p = p0 + min(tid & 31, np - 1);
-    return a.pair_tok ? a.pair_tok[p] : p;
-  }();
-  struct BRegs {
-    i32x4 v[4];
-    float x, s;
-  };
-  auto load_b = [&](int sbk, BRegs& br) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      br.v[j] = *(const __attribute__((address_space(1))) i32x4*)(bsrc[j] + (size_t)sbk * 256);
-    br.x = a.bx[(size_t)xrow * (a.K >> 5) + sbk * 8 + (tid & 7)];
-    br.s = a.bs[(size_t)srow * nsb + sbk];
-  };
-  auto store_b = [&](const BRegs& br, int buf) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      *reinterpret_cast<uint64_t*>(&bst[buf][0] + bdst0[j]) =
-          ((uint64_t)(uint32_t)br.v[j][1] << 32) | (uint32_t)br.v[j][0];
-      *reinterpret_cast<uint64_t*>(&bst[buf][0] + bdst1[j]) =
-          ((uint64_t)(uint32_t)br.v[j][3] << 32) | (uint32_t)br.v[j][2];
+    for (int c = 0; c < kPW; ++c) {
+      const int pg = (wave * kPW + c) % PG;
+      brow[c] = pg < NPG ? (uint32_t)row_of(16 * pg + lr) * ib + 16 * lp : (uint32_t)kPast;
     }
-    bsx[buf][xdst] = br.x;
-    if (tid < kQPairs) bss[buf][tid] = br.s;
-  };
-  struct ARegs {
-    i32x4 v[3];
-  };
-  auto load_a = [&](int sbk, ARegs& ar) {
-#pragma unroll
-    for (int it = 0; it < 3; ++it)
-      if (it < 2 || lane < 16)
-        ar.v[it] = *(const __attribute__((address_space(1))) i32x4*)(asrc[it] + (size_t)sbk * 144);
-  };
-  auto store_a = [&](const ARegs& ar) {  // the wave's slice: its reads of the last super-block are done
-#pragma unroll
-    for (int it = 0; it < 3; ++it)
-      if (it < 2 || lane < 16) *reinterpret_cast<i32x4*>(&ast[wave][adst[it]]) = ar.v[it];
-  };
-  // header of row i (lanes g == 0, from the wave's slice) -> LDS: d, dmin*m_j (the reference's f32
-  // products), sc_j
-  auto decode_hdr = [&]() {
-    if (g == 0) {
-      const i32x4 hdr = *reinterpret_cast<const i32x4*>(&ast[wave][i * 144]);
-      const uint32_t dd = (uint32_t)hdr[0];
-      const uint32_t s3[3] = {(uint32_t)hdr[1], (uint32_t)hdr[2], (uint32_t)hdr[3]};
-      const float d = h2f(dd & 0xFFFFu), dmin = h2f(dd >> 16);
-      hd[wave][i] = d;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        uint32_t sc, mm;
-        q4k_scale_min((uint32_t)j, s3, sc, mm);
-        hsc[wave][j][i] = (int)sc;
-        hm[wave][(j >> 2) * 64 + 16 * (j & 3) + i] = dmin * (float)mm;
+    // (K step, term) of the pieces: kPW <= PG pieces share one, or each has its own (PG = 1)
+    auto bkt = [&](int c) { return (uint32_t)((wave * kPW + c) / PG) * 64u; };
+    // the sub-block sums: PG = 1: the lane's own operand; else waves 0 .. NPG-1 bring those of
+    // pair group `wave`
+    const uint32_t xrow = PG == 1 ? (uint32_t)row_of(i) * ib + 1024 + 16 * g
+                          : wave < NPG ? (uint32_t)row_of(16 * wave + lr) * ib + 1024 + 16 * lp : (uint32_t)kPast;
+    const uint32_t prow = GATEUP ? (uint32_t)row_of(tid & (kPairs - 1)) : (uint32_t)((row_of(tid & (kPairs - 1))) * nsb);
+    const float* pbase = GATEUP ? q.pinv : q.pinv + (size_t)p0 * nsb;
+    if (tid < kPairs) {
+      if (GATEUP) {
+        pst[0][tid] = pbase[prow];
+        pw[tid] = sh ? 1.f : a.pair_w[p0 + min(tid, np - 1)];
       }
     }
-  };
+    i32x4 bR[kPW], xR = {0, 0, 0, 0};
+    float pR = 0.f;
+    auto load_x = [&](int sb) {
+      xR = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(xb, (int)xrow, sb * kQImgSb, 0));
+    };
+    auto load_b = [&](int sb, int s) {
+#pragma unroll
+      for (int c = 0; c < kPW; ++c)
+        bR[c] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                               xb, (int)brow[c], (int)(bkt(c) + (uint32_t)(sb * kQImgSb + s * (kKS * 128))), 0));
+      if (s == 0) {
+        if (PG > 1) load_x(sb);
+        if (!GATEUP) pR = pbase[prow + (uint32_t)sb];
+      }
+    };
+    auto store_b = [&](int sb, int s, int buf) {
+#pragma unroll
+      for (int c = 0; c < kPW; ++c)
+        *reinterpret_cast<i32x4*>(&lds[buf * kStage + (wave * kPW + c) * 1024 + bwr]) = bR[c];
+      if (s == 0) {
+        if (PG > 1 && wave < NPG) *reinterpret_cast<i32x4*>(&xst[sb & 1][wave * 1024 + bwr]) = xR;
+        if (!GATEUP) pst[sb & 1][tid & (kPairs - 1)] = pR;
+      }
+    };
+    // Weight loads are issued for every half super-block and one past the last, where nothing is
+    // fetched.
+    i32x4 aR[kPF][NT], hR;
+    auto load_hdr = [&](int sb) {
+      hR = *(const __attribute__((address_space(1))) i32x4*)(hsrc + (uint32_t)(min(sb, nsb - 1) * 144));
+    };
+    auto load_a = [&](int sb, int half) {
+      const int off = aoff + 64 * half + (sb < nsb ? 0 : kPast);
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        aR[half % kPF][t] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                          GATEUP && t >= kTM ? wb1 : wb0, off, (int)wt[t] + sb * 144, 0));
+    };
+    load_b(0, 0);
+    load_hdr(0);
+    load_a(0, 0);
+    if (kPF == 2) load_a(0, 1);
 
-  f32x4 acc[2];
-  acc[0] = acc[1] = f32x4{0.f, 0.f, 0.f, 0.f};
-  BRegs bR;
-  ARegs aR;
-  load_b(0, bR);
-  load_a(0, aR);
-  for (int sbk = 0; sbk < nsb; ++sbk) {
-    const int buf = sbk & 1;
-    store_b(bR, buf);  // buffer buf was last read in super-block sbk-2, before the last barrier
-    store_a(aR);
-    decode_hdr();      // this wave's header slots were last read before the last barrier
-    __syncthreads();   // the stages of super-block sbk and the headers are in LDS
-    if (sbk + 1 < nsb) {
-      load_b(sbk + 1, bR);
-      load_a(sbk + 1, aR);
-    }
-    if (tile_in) {
-      const uint8_t* bb = &bst[buf][0];
-      int I0[2][4], I1[2][4];
+    const uint32_t psel = 0x07000700u | (uint32_t)(g & 2) | (uint32_t)((g & 2) + 1) << 16;  // v_perm: bytes {s, 0x64} twice
+    f32x4 acc[NT][NPG];
 #pragma unroll
-      for (int pg = 0; pg < 2; ++pg)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) I0[pg][r] = I1[pg][r] = 0;
+      for (int pg = 0; pg < NPG; ++pg) acc[t][pg] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    for (int sb = 0; sb < nsb; ++sb) {
+      const f16x2 k1024 = {(_Float16)-1024.f, (_Float16)-1024.f};
+      auto as2 = [](uint32_t u) { return __builtin_bit_cast(f16x2, u); };
+      f32x4 S[NT][NPG];
+      i32x4 raw[NT];
+      f16x2 sc_lo[NT], sc_hi[NT];
+      // half a super-block: its weights, and the scales of the lane's two sub-blocks
+      auto begin_half = [&](int half) {
+        // (the wave's own LDS accesses stay in order)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        // A: elements [8g, 8g+8) of sub-block j of row i as int8 (low nibbles: even j)
-        const uint64_t qb = *reinterpret_cast<const uint64_t*>(&ast[wave][i * 144 + 16 + 32 * (j >> 1) + 8 * g]);
-        const uint32_t lo = (uint32_t)qb, hi = (uint32_t)(qb >> 32);
-        const uint32_t sh = (j & 1) * 4;
-        const long av = (long)(((uint64_t)((hi >> sh) & 0x0F0F0F0Fu) << 32) | ((lo >> sh) & 0x0F0F0F0Fu));
-        const i32x4v scv = *reinterpret_cast<const i32x4v*>(&hsc[wave][j][4 * g]);
-        const int slot = (lane ^ (2 * j)) * 8;
+        for (int t = 0; t < NT; ++t) *reinterpret_cast<i32x4*>(&ast[wave][t * 1024 + awr]) = aR[half % kPF][t];
+        if (half == 0) *reinterpret_cast<i32x4*>(&hst[wave][(lane % (16 * NT)) * 16]) = hR;
+        if (PG == 1 && half) load_x(sb);
+        if (kPF == 2)
+          load_a(sb + 1, half);
+        else
+          load_a(half ? sb + 1 : sb, half ^ 1);
+        if (half == 0) load_hdr(sb + 1);
 #pragma unroll
-        for (int pg = 0; pg < 2; ++pg) {
-          const long bv0 = *reinterpret_cast<const long*>(bb + ((0 * 2 + pg) * 8 + j) * 512 + slot);
-          const long bv1 = *reinterpret_cast<const long*>(bb + ((1 * 2 + pg) * 8 + j) * 512 + slot);
-          const i32x4v z = {0, 0, 0, 0};
-          const i32x4v d0 = __builtin_amdgcn_mfma_i32_16x16x32_i8(av, bv0, z, 0, 0, 0);
-          const i32x4v d1 = __builtin_amdgcn_mfma_i32_16x16x32_i8(av, bv1, z, 0, 0, 0);
+        for (int t = 0; t < NT; ++t) {
+          raw[t] = *reinterpret_cast<const i32x4*>(&ast[wave][t * 1024 + ard]);
+          const i32x4 hw = *reinterpret_cast<const i32x4*>(&hst[wave][t * 256 + i * 16]);
+          const uint32_t w0 = (uint32_t)hw[1], w2 = (uint32_t)hw[3];
+          const uint32_t sw = half ? (w2 & 0x0F0F0F0Fu) | ((w0 >> 2) & 0x30303030u) : w0 & 0x3F3F3F3Fu;
+          // bytes 2 (g / 2), + 1: the scales of sub-blocks 4 half + these, as f16 1024 + sc, then
+          // 2^10 sc and, for nibbles left in place (16 q), 2^6 sc
+          const f16x2 s2 = (as2(__builtin_amdgcn_perm(0x64646464u, sw, psel)) + k1024) * f16x2{(_Float16)1024.f, (_Float16)64.f};
+          sc_lo[t] = __builtin_shufflevector(s2, s2, 0, 0);
+          sc_hi[t] = __builtin_shufflevector(s2, s2, 1, 1);
+        }
+      };
+#pragma unroll
+      for (int s = 0; s < kNS; ++s) {
+        const int buf = (sb * kNS + s) & 1;
+        if (s * kKS % 4 == 0) begin_half(s * kKS / 4);
+        store_b(sb, s, buf);  // last read two stages ago, before the previous barrier
+        __syncthreads();
+        if (s + 1 < kNS)
+          load_b(sb, s + 1);
+        else
+          load_b(min(sb + 1, nsb - 1), 0);
+        // The stage's K steps. Each fragment is read from LDS two fragments ahead; with two waves
+        // per SIMD (NT = 4), step ks + 1's weights are unpacked among step ks's MFMAs.
+        constexpr int kWB = NT == 4 ? 2 : 1;  // unpacked K steps in registers
+        f16x8 wf[kWB][NT], xf[3];
+        auto unpack = [&](int n, f16x8 (&o)[NT]) {
+          const int u = (n >> 1) & 1, hl = n & 1;
+#pragma unroll
+          for (int t = 0; t < NT; ++t) {
+            const uint32_t x0 = (uint32_t)raw[t][2 * u], x1 = (uint32_t)raw[t][2 * u + 1];
+            const uint32_t msk = hl ? 0x00F000F0u : 0x000F000Fu;
+            const f16x2 sc = hl ? sc_hi[t] : sc_lo[t];
+            const f16x2 a0 = as2(x0 & msk) * sc, a1 = as2((x0 >> 8) & msk) * sc;
+            const f16x2 a2 = as2(x1 & msk) * sc, a3 = as2((x1 >> 8) & msk) * sc;
+            o[t] = f16x8{a0.x, a0.y, a1.x, a1.y, a2.x, a2.y, a3.x, a3.y};
+          }
+        };
+        constexpr int kF = 2 * NPG;  // fragments (term, pair group) per K step
+        auto frag = [&](int f) {     // f: fragment of the stage
+          return *reinterpret_cast<const f16x8*>(
+              &lds[buf * kStage + ((f / kF * 2 + f % kF / NPG) * PG + f % NPG) * 1024 + brd]);
+        };
+        xf[0] = frag(0);
+        xf[1] = frag(1);
+        if constexpr (kWB == 2) unpack(s * kKS, wf[0]);
+#pragma unroll
+        for (int f = 0; f < kKS * kF; ++f) {
+          const int ks = f / kF, pg = f % NPG;
+          if (f + 2 < kKS * kF) xf[(f + 2) % 3] = frag(f + 2);
+          if constexpr (kWB == 2) {
+            if (f % kF == 0 && ks + 1 < kKS) unpack(s * kKS + ks + 1, wf[(ks + 1) & 1]);
+          } else {
+            if (kKS == 8 && f == 4 * kF) begin_half(1);
+            if (f % kF == 0) unpack(s * kKS + ks, wf[0]);
+          }
+#pragma unroll
+          for (int t = 0; t < NT; ++t) {
+            const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+            S[t][pg] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[f % 3], wf[ks & (kWB - 1)][t],
+                                                              s == 0 && f < NPG ? z : S[t][pg], 0, 0, 0);
+          }
+          if constexpr (kWB == 2) {
+            if (f + 2 < kKS * kF) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, NT, 0);
+            if (ks + 1 < kKS) __builtin_amdgcn_sched_group_barrier(0x002, (72 + kF - 1) / kF, 0);
+          } else {
+            if (f % kF == kF - 1) __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      // acc += (d S - dmin M) (down: / p): M is the min term's MFMA, the eight mins of row i as
+      // f16 in image order in every lane group against the sums' terms
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const i32x4 hw = *reinterpret_cast<const i32x4*>(&hst[wave][t * 256 + i * 16]);
+        const uint32_t dd = (uint32_t)hw[0], w1 = (uint32_t)hw[2], w2 = (uint32_t)hw[3];
+        const float dv = 16384.f * (float)__builtin_bit_cast(_Float16, (uint16_t)dd);  // the weights are 2^-14 sc q
+        const float dm = -32.f * (float)__builtin_bit_cast(_Float16, (uint16_t)(dd >> 16));  // the sums are 2^-5 X
+        const uint32_t m03 = w1 & 0x3F3F3F3Fu, m47 = ((w2 >> 4) & 0x0F0F0F0Fu) | ((w1 >> 2) & 0x30303030u);
+        auto m2 = [&](uint32_t m, uint32_t sel) { return as2(__builtin_amdgcn_perm(0x64646464u, m, sel)) + k1024; };
+        const f16x2 ma = m2(m03, 0x07020700u), mb = m2(m03, 0x07030701u), mc = m2(m47, 0x07020700u), md = m2(m47, 0x07030701u);
+        const f16x8 mf = {ma.x, ma.y, mb.x, mb.y, mc.x, mc.y, md.x, md.y};
+#pragma unroll
+        for (int pg = 0; pg < NPG; ++pg) {
+          const f16x8 xf = PG == 1 ? __builtin_bit_cast(f16x8, xR)
+                                   : *reinterpret_cast<const f16x8*>(&xst[sb & 1][pg * 1024 + brd]);
+          const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+          const f32x4 m = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf, mf, z, 0, 0, 0);
+          f32x4 pv = {1.f, 1.f, 1.f, 1.f};
+          if (!GATEUP) pv = *reinterpret_cast<const f32x4*>(&pst[sb & 1][16 * pg + 4 * g]);
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            I0[pg][r] += __mul24(scv[r], d0[r]);
-            I1[pg][r] += __mul24(scv[r], d1[r]);
+            if (GATEUP)
+              acc[t][pg][r] = __builtin_fmaf(dm, m[r], __builtin_fmaf(dv, S[t][pg][r], acc[t][pg][r]));
+            else
+              acc[t][pg][r] = __builtin_fmaf(__builtin_fmaf(dm, m[r], dv * S[t][pg][r]), pv[r], acc[t][pg][r]);
           }
         }
       }
-      // min term: [16 rows x 8 sub-blocks] x [8 sub-blocks x 16 pairs] per pair group
-      f32x4 Mn[2];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+
+    if constexpr (!GATEUP) {
 #pragma unroll
-      for (int pg = 0; pg < 2; ++pg) {
-        Mn[pg] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int t = 0; t < NT; ++t) {
+        const int row = wrow0 + 16 * t + i;
+        if (row >= M) continue;
 #pragma unroll
-        for (int c = 0; c < 2; ++c)
-          Mn[pg] = __builtin_amdgcn_mfma_f32_16x16x4f32(hm[wave][c * 64 + lane], bsx[buf][(pg * 2 + c) * 64 + lane],
-                                                        Mn[pg], 0, 0, 0);
+        for (int pg = 0; pg < NPG; ++pg)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int pl = 16 * pg + 4 * g + r;
+            if (pl < np) q.out[(size_t)(p0 + pl) * M + row] = acc[t][pg][r];
+          }
       }
-      const f32x4 dv = *reinterpret_cast<const f32x4*>(&hd[wave][4 * g]);
+    } else {
+      // h = act(gate + b_g, up + b_u) x routing weight in registers (this lane: rows 16 t + i of
+      // the wave's, pairs 4g + r of each group), then the item's 256 rows of a pair, one
+      // super-block, are split. Largest magnitudes and sums go over the
+      // 16 lanes of a row group, the magnitudes over the waves through LDS; the halves are put
+      // in place in LDS and leave as whole 16-byte pieces.
+      float hv[kTM][NPG][4], hsum[NPG][4];
 #pragma unroll
-      for (int pg = 0; pg < 2; ++pg) {
-        const float s = bss[buf][pg * 16 + i];
+      for (int t = 0; t < kTM; ++t) {
+        const int row = wrow0 + 16 * t + i;
+        const float bg = !sh && q.b0 ? q.b0[(size_t)e * M + row] : 0.f, bu = !sh && q.b1 ? q.b1[(size_t)e * M + row] : 0.f;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float v = __builtin_fmaf((float)I1[pg][r], 0.0078125f, (float)I0[pg][r]);  // A0 + A1/128
-          acc[pg][r] = __builtin_fmaf(dv[r] * s, v, acc[pg][r]) - Mn[pg][r];
+        for (int pg = 0; pg < NPG; ++pg) {
+          const f32x4 pv = *reinterpret_cast<const f32x4*>(&pst[0][16 * pg + 4 * g]);
+          const f32x4 rw = *reinterpret_cast<const f32x4*>(&pw[16 * pg + 4 * g]);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float gv = __builtin_fmaf(acc[t][pg][r], pv[r], bg), uv = __builtin_fmaf(acc[kTM + t][pg][r], pv[r], bu);
+            hv[t][pg][r] = (q.act == MR_ACT_SWIGLU_OAI ? swiglu_oai(gv, uv, a.alpha, a.limit) : silu_mul(gv, uv)) * rw[r];
+          }
         }
       }
-    }
-  }
-  if (GATEUP) {
-    __syncthreads();  // every wave is done with the stages: reuse them for the gate/up tiles
-    float* ep = reinterpret_cast<float*>(&bst[0][0]);  // [mat][32 rows][32 pairs]
 #pragma unroll
-    for (int pg = 0; pg < 2; ++pg)
+      for (int pg = 0; pg < NPG; ++pg)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) ep[(m * 32 + (wave & 1) * 16 + 4 * g + r) * kQPairs + pg * 16 + i] = acc[pg][r];
-    __syncthreads();
-    const int r0 = rt * kRows;
-    for (int q = tid; q < 32 * kQPairs; q += 256) {
-      const int pl = q >> 5, rr = q & 31;  // consecutive threads: consecutive rows of one pair
-      const int row = r0 + rr;
-      if (pl >= np || row >= a.M) continue;
-      float gv = ep[rr * kQPairs + pl], uv = ep[(32 + rr) * kQPairs + pl];
-      if (a.b0) gv = gv + a.b0[(size_t)e * a.M + row];
-      if (a.b1) uv = uv + a.b1[(size_t)e * a.M + row];
-      const float h = a.act == MR_ACT_SWIGLU_OAI ? swiglu_oai(gv, uv, a.alpha, a.limit) : silu_mul(gv, uv);
-      a.out[(size_t)(p0 + pl) * a.M + row] = h * pw[pl];
-    }
-  } else if (tile_in) {
+        for (int r = 0; r < 4; ++r) {
+          float m = fmaxf(fabsf(hv[0][pg][r]), fabsf(hv[kTM - 1][pg][r])), s = kTM == 2 ? hv[0][pg][r] + hv[kTM - 1][pg][r] : hv[0][pg][r];
+          m = fmaxf(m, dpp_f<kDppXor1>(m)), s += dpp_f<kDppXor1>(s);
+          m = fmaxf(m, dpp_f<kDppXor2>(m)), s += dpp_f<kDppXor2>(s);
+          m = fmaxf(m, dpp_f<kDppHMirror>(m)), s += dpp_f<kDppHMirror>(s);
+          m = fmaxf(m, dpp_f<kDppMirror>(m)), s += dpp_f<kDppMirror>(s);
+          hsum[pg][r] = s;
+          if (i == 0) {
+            wred[wave][16 * pg + 4 * g + r] = m;
+            if (NT == 2) wsum[wave][16 * pg + 4 * g + r] = s;  // half a sub-block
+          }
+        }
+      __syncthreads();  // the magnitudes are in place and every wave is done with the stages
+      // element 16 el + i of the super-block, el = kTM wave + t: sub-block el / 2, i.e. h = el / 8,
+      // g = 2 (el / 4 % 2) + el % 2, hl = el / 2 % 2, u = i / 8
+      auto at = [&](int el) {
+        return (4 * (el >> 3) + 2 * (i >> 3) + ((el >> 1) & 1)) * 128 + ((el >> 1) & 2) * 16 + (el & 1) * 16 + kQPerm[i & 7] * 2;
+      };
 #pragma unroll
-    for (int pg = 0; pg < 2; ++pg) {
-      const int pl = pg * 16 + i;
-      if (pl < np && wrow0 + 4 * g < a.M)
-        *reinterpret_cast<f32x4*>(a.out + (size_t)(p0 + pl) * a.M + wrow0 + 4 * g) = acc[pg];
+      for (int pg = 0; pg < NPG; ++pg) {
+        f32x4 m4 = *reinterpret_cast<const f32x4*>(&wred[0][16 * pg + 4 * g]);
+#pragma unroll
+        for (int v = 1; v < NW; ++v) {
+          const f32x4 o4 = *reinterpret_cast<const f32x4*>(&wred[v][16 * pg + 4 * g]);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) m4[r] = fmaxf(m4[r], o4[r]);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int pl = 16 * pg + 4 * g + r;
+          float p, pinv;
+          pow2_scale(m4[r], p, pinv);
+          uint8_t* im = &lds[pl * kEpRow];
+#pragma unroll
+          for (int t = 0; t < kTM; ++t) {
+            uint32_t h, l;
+            split2(hv[t][pg][r] * p, h, l);
+            uint8_t* d = im + at(kTM * wave + t);
+            *reinterpret_cast<uint16_t*>(d) = (uint16_t)h;
+            *reinterpret_cast<uint16_t*>(d + 64) = (uint16_t)l;
+          }
+          const int sub = kTM * wave / 2;  // its sums: NT = 2: with the next wave's half
+          if (i < 4 && (kTM == 2 || wave % 2 == 0)) {
+            const float X = NT == 2 ? hsum[pg][r] + wsum[(NW > 1 ? wave + 1 : 0) % NW][pl] : hsum[pg][r];
+            *reinterpret_cast<uint16_t*>(im + 1024 + i * 16 + kQPerm[sub] * 2) = (uint16_t)sum_term(X * p, i);
+          }
+          if (wave == 0 && i == 0 && pl < np) q.hpinv[(size_t)(p0 + pl) * (M >> 8) + rt] = pinv;
+        }
+      }
+      __syncthreads();
+      constexpr int kPieces = kQImgSb / 16;
+      for (int c = tid; c < np * kPieces; c += NW * 64) {
+        const int pl = c / kPieces, o = (c - pl * kPieces) * 16;
+        *reinterpret_cast<i32x4*>(q.himg + ((size_t)(p0 + pl) * (M >> 8) + rt) * kQImgSb + o) =
+            *reinterpret_cast<const i32x4*>(&lds[pl * kEpRow + o]);
+      }
     }
+  };
+  if constexpr (PG == 1) {
+    run(std::integral_constant<int, 1>{});
+  } else {
+    static_assert(PG == 4, "pair tiles of 16 or 64");
+    const int npg = (np + 15) >> 4;
+    if (npg == 4) run(std::integral_constant<int, 4>{});
+    else if (npg == 3) run(std::integral_constant<int, 3>{});
+    else if (npg == 2) run(std::integral_constant<int, 2>{});
+    else run(std::integral_constant<int, 1>{});
   }
 }
 
@@ -362,23 +578,13 @@ __global__ __launch_bounds__(256, 3) void k_grouped_q4k(GQ4Args a) {
 namespace {
 constexpr uint64_t kQAlign = 256;
 uint64_t qup(uint64_t v) { return (v + kQAlign - 1) / kQAlign * kQAlign; }
-struct TermsPlan {
-  uint64_t t0, t1, s, x, total;
-};
-TermsPlan terms_plan(uint64_t rows, uint64_t D, uint64_t o) {
-  TermsPlan p{};
-  p.t0 = o, o += qup(rows * D);
-  p.t1 = o, o += qup(rows * D);
-  p.s = o, o += qup(rows * (D / 256) * 4);
-  p.x = o, o += qup(rows * (D / 32) * 4);
-  p.total = o;
-  return p;
-}
+uint64_t img_bytes(uint64_t rows, uint64_t D) { return rows * (D / 256) * kQImgSb; }
 struct Q4Plan {
-  uint64_t pair_tok, pair_w, pair_of, exp_off, tile_off;
-  TermsPlan xt, ht, hst;
-  uint64_t h, o, hsh, osh, sig, total;
+  uint64_t pair_tok, pair_w, pair_of, exp_off, tile_off, tile_exp, hist;
+  uint64_t xp, himg, hp, hsimg, hsp, xo, osh, sig, total;
 };
+// The x images are last read by the gate/up launch and o is first written by the down launch:
+// they share xo.
 Q4Plan q4_plan(uint64_t T, uint64_t k, uint64_t E, uint64_t I, uint64_t H, uint64_t Ish) {
   Q4Plan p{};
   const uint64_t P = T * k;
@@ -388,35 +594,20 @@ Q4Plan q4_plan(uint64_t T, uint64_t k, uint64_t E, uint64_t I, uint64_t H, uint6
   p.pair_of = o, o += qup(P * 4);
   p.exp_off = o, o += qup((E + 1) * 4);
   p.tile_off = o, o += qup((E + 1) * 4);
-  p.xt = terms_plan(T, H, o), o = p.xt.total;
-  p.h = o, o += qup(P * I * 4);
-  p.ht = terms_plan(P, I, o), o = p.ht.total;
-  p.o = o, o += qup(P * H * 4);
+  p.tile_exp = o, o += qup(group_tiles_max(P, E, kGroupTileMin) * 4);
+  p.hist = o, o += qup(group_hist_bytes(P, E));
+  p.xp = o, o += qup(T * 4);
+  p.himg = o, o += qup(img_bytes(P, I));
+  p.hp = o, o += qup(P * (I / 256) * 4);
+  p.xo = o, o += qup(std::max(img_bytes(T, H), P * H * 4));
   if (Ish) {
-    p.hsh = o, o += qup(T * Ish * 4);
-    p.hst = terms_plan(T, Ish, o), o = p.hst.total;
+    p.hsimg = o, o += qup(img_bytes(T, Ish));
+    p.hsp = o, o += qup(T * (Ish / 256) * 4);
     p.osh = o, o += qup(T * H * 4);
     p.sig = o, o += qup(T * 4);
   }
   p.total = o;
   return p;
-}
-struct Terms {
-  int8_t* t0;
-  int8_t* t1;
-  float* s;
-  float* x;
-};
-Terms terms_at(char* b, const TermsPlan& p) {
-  return Terms{reinterpret_cast<int8_t*>(b + p.t0), reinterpret_cast<int8_t*>(b + p.t1),
-               reinterpret_cast<float*>(b + p.s), reinterpret_cast<float*>(b + p.x)};
-}
-hipError_t split(const Launch& K, const float* src, uint64_t rows, uint32_t D, const Terms& t) {
-  const uint64_t items = rows * (D / 256);
-  ProfScope ps(K, "split_q4k");
-  hipLaunchKernelGGL(k_split_q4k, dim3((unsigned)((items + 3) / 4)), dim3(256), 0, K.s, src, (int)rows, (int)D, t.t0,
-                     t.t1, t.s, t.x);
-  return hipGetLastError();
 }
 }  // namespace
 
@@ -442,71 +633,81 @@ bool grouped_q4k_supported(const mr_layer& L) {
 hipError_t launch_grouped_q4k(const Launch& K, const mr_layer& L, const float* x, uint32_t T, const int32_t* idx,
                               const float* w, float* y, void* scratch) {
   const int k = (int)L.d.top_k, E = (int)L.E, H = (int)L.H, I = (int)L.I, Ish = L.d.sh_gate ? (int)L.Ish : 0;
+  // The kernels address the images of a call's rows within kPast bytes: more tokens than that
+  // holds run in parts (a token's result depends on that token alone).
+  const uint32_t T_max = (uint32_t)((uint64_t)kPast / img_bytes(1, (uint64_t)H));
+  if (T > T_max) {
+    for (uint32_t t0 = 0; t0 < T; t0 += T_max) {
+      const hipError_t e = launch_grouped_q4k(K, L, x + (size_t)t0 * H, std::min(T_max, T - t0), idx + (size_t)t0 * k,
+                                              w + (size_t)t0 * k, y + (size_t)t0 * H, scratch);
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+  }
   const int P = (int)T * k;
   const Q4Plan p = q4_plan(T, k, E, I, H, Ish);
   char* b = static_cast<char*>(scratch);
-  int32_t* pair_tok = reinterpret_cast<int32_t*>(b + p.pair_tok);
-  float* pair_w = reinterpret_cast<float*>(b + p.pair_w);
-  int32_t* pair_of = reinterpret_cast<int32_t*>(b + p.pair_of);
-  int32_t* exp_off = reinterpret_cast<int32_t*>(b + p.exp_off);
-  int32_t* tile_off = reinterpret_cast<int32_t*>(b + p.tile_off);
-  const Terms xt = terms_at(b, p.xt), ht = terms_at(b, p.ht);
-  float* h = reinterpret_cast<float*>(b + p.h);
-  float* o = reinterpret_cast<float*>(b + p.o);
+  auto f32_at = [&](uint64_t o) { return reinterpret_cast<float*>(b + o); };
+  auto i32_at = [&](uint64_t o) { return reinterpret_cast<int32_t*>(b + o); };
+  auto u8_at = [&](uint64_t o) { return reinterpret_cast<uint8_t*>(b + o); };
+  // Pairs per tile: 16 while the experts' mean is at most 8, so that few experts need a second
+  // tile (which reads the expert's weights again), else 64: the 16-pair kernels keep twice the
+  // weight bytes in flight (128 pairs of 128 experts: gate/up 50 against 75 us, 3,840 of 512: 225
+  // against 303), and past 16 pairs every further tile costs them what the first did.
+  const bool small = (uint64_t)P <= 8ull * (uint64_t)E;
+  const int tile = small ? 16 : 64;
+  const GroupOut go{i32_at(p.pair_tok), f32_at(p.pair_w),   i32_at(p.pair_of), i32_at(p.exp_off),
+                    i32_at(p.tile_off), i32_at(p.tile_exp), i32_at(p.hist)};
   hipError_t e;
-  if ((e = launch_group(K, idx, w, P, k, E, pair_tok, pair_w, pair_of, exp_off, tile_off)) != hipSuccess) return e;
-  if ((e = split(K, x, T, (uint32_t)H, xt)) != hipSuccess) return e;
-  const int max_tiles = (P + kQPairs - 1) / kQPairs + E;
+  if ((e = launch_group(K, idx, w, P, k, E, tile, go)) != hipSuccess) return e;
+  float* sig = Ish ? f32_at(p.sig) : nullptr;
+  {
+    ProfScope ps(K, "split_q4k");
+    hipLaunchKernelGGL(k_split_f16, dim3(T), dim3(256), 0, K.s, x, H, u8_at(p.xo), f32_at(p.xp),
+                       Ish ? L.d.sh_gate_inp : nullptr, sig);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
+  const uint64_t tiles = group_tiles_max(P, E, tile), sh_tiles = Ish ? (T + tile - 1) / tile : 0;
   GQ4Args a{};
-  a.w0 = expert_loc(L.d.gate), a.w1 = expert_loc(L.d.up), a.b0 = L.d.gate_bias, a.b1 = L.d.up_bias;
-  a.t0 = xt.t0, a.t1 = xt.t1, a.bs = xt.s, a.bx = xt.x;
-  a.pair_tok = pair_tok, a.pair_w = pair_w, a.exp_off = exp_off, a.tile_off = tile_off;
-  a.out = h, a.M = I, a.K = H, a.E = E, a.act = (int)L.d.act, a.alpha = L.d.alpha, a.limit = L.d.limit;
+  a.r.w0 = expert_loc(L.d.gate), a.r.w1 = expert_loc(L.d.up), a.r.b0 = L.d.gate_bias, a.r.b1 = L.d.up_bias;
+  a.r.img = u8_at(p.xo), a.r.pinv = f32_at(p.xp), a.r.himg = u8_at(p.himg), a.r.hpinv = f32_at(p.hp);
+  a.r.M = I, a.r.K = H, a.r.act = (int)L.d.act;
+  if (Ish) {
+    a.s.w0 = expert_loc(L.d.sh_gate), a.s.w1 = expert_loc(L.d.sh_up);
+    a.s.img = a.r.img, a.s.pinv = a.r.pinv, a.s.himg = u8_at(p.hsimg), a.s.hpinv = f32_at(p.hsp);
+    a.s.M = Ish, a.s.K = H, a.s.act = MR_ACT_SILU;
+    a.sh_T = (int)T;
+  }
+  a.pair_tok = go.pair_tok, a.pair_w = go.pair_w, a.exp_off = go.exp_off, a.tile_off = go.tile_off, a.tile_exp = go.tile_exp;
+  a.E = E, a.alpha = L.d.alpha, a.limit = L.d.limit;
   {
     ProfScope ps(K, "grouped_q4k_gateup");
-    hipLaunchKernelGGL(k_grouped_q4k<true>, dim3(grouped_grid((uint64_t)((I + 31) / 32) * max_tiles)), dim3(256), 0, K.s, a);
+    const dim3 grid(grouped_grid((uint64_t)(I / 256) * tiles + (uint64_t)(Ish / 256) * sh_tiles));
+    if (small)
+      hipLaunchKernelGGL((k_grouped_q4k<true, 1>), grid, dim3(64 * q4_waves(true, 1)), 0, K.s, a);
+    else
+      hipLaunchKernelGGL((k_grouped_q4k<true, 4>), grid, dim3(64 * q4_waves(true, 4)), 0, K.s, a);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
-  if ((e = split(K, h, (uint64_t)P, (uint32_t)I, ht)) != hipSuccess) return e;
   GQ4Args d{};
-  d.w0 = expert_loc(L.d.down);
-  d.t0 = ht.t0, d.t1 = ht.t1, d.bs = ht.s, d.bx = ht.x;
-  d.exp_off = exp_off, d.tile_off = tile_off, d.out = o, d.M = H, d.K = I, d.E = E;
+  d.r.w0 = expert_loc(L.d.down);
+  d.r.img = u8_at(p.himg), d.r.pinv = f32_at(p.hp), d.r.out = f32_at(p.xo), d.r.M = H, d.r.K = I;
+  if (Ish) {
+    d.s.w0 = expert_loc(L.d.sh_down);
+    d.s.img = u8_at(p.hsimg), d.s.pinv = f32_at(p.hsp), d.s.out = f32_at(p.osh), d.s.M = H, d.s.K = Ish;
+    d.sh_T = (int)T;
+  }
+  d.exp_off = go.exp_off, d.tile_off = go.tile_off, d.tile_exp = go.tile_exp, d.E = E;
   {
     ProfScope ps(K, "grouped_q4k_down");
-    hipLaunchKernelGGL(k_grouped_q4k<false>, dim3(grouped_grid((uint64_t)((H + 63) / 64) * max_tiles)), dim3(256), 0, K.s, d);
+    const dim3 grid(grouped_grid((uint64_t)((H + 255) / 256) * (tiles + sh_tiles)));
+    if (small)
+      hipLaunchKernelGGL((k_grouped_q4k<false, 1>), grid, dim3(64 * q4_waves(false, 1)), 0, K.s, d);
+    else
+      hipLaunchKernelGGL((k_grouped_q4k<false, 4>), grid, dim3(64 * q4_waves(false, 4)), 0, K.s, d);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
-  float* osh = nullptr;
-  float* sig = nullptr;
-  if (Ish) {  // the shared expert: one expert over all T tokens, weight 1, then its sigmoid gate
-    float* hsh = reinterpret_cast<float*>(b + p.hsh);
-    const Terms hst = terms_at(b, p.hst);
-    osh = reinterpret_cast<float*>(b + p.osh);
-    sig = reinterpret_cast<float*>(b + p.sig);
-    const int tiles = ((int)T + kQPairs - 1) / kQPairs;
-    GQ4Args s{};
-    s.w0 = expert_loc(L.d.sh_gate), s.w1 = expert_loc(L.d.sh_up);
-    s.t0 = xt.t0, s.t1 = xt.t1, s.bs = xt.s, s.bx = xt.x;
-    s.single_p = (int)T, s.out = hsh, s.M = Ish, s.K = H, s.E = 1, s.act = MR_ACT_SILU;
-    {
-      ProfScope ps(K, "grouped_q4k_shared_gateup");
-      hipLaunchKernelGGL(k_grouped_q4k<true>, dim3(grouped_grid((uint64_t)((Ish + 31) / 32) * tiles)), dim3(256), 0, K.s, s);
-      if ((e = hipGetLastError()) != hipSuccess) return e;
-    }
-    if ((e = split(K, hsh, T, (uint32_t)Ish, hst)) != hipSuccess) return e;
-    GQ4Args sd{};
-    sd.w0 = expert_loc(L.d.sh_down);
-    sd.t0 = hst.t0, sd.t1 = hst.t1, sd.bs = hst.s, sd.bx = hst.x;
-    sd.single_p = (int)T, sd.out = osh, sd.M = H, sd.K = Ish, sd.E = 1;
-    {
-      ProfScope ps(K, "grouped_q4k_shared_down");
-      hipLaunchKernelGGL(k_grouped_q4k<false>, dim3(grouped_grid((uint64_t)((H + 63) / 64) * tiles)), dim3(256), 0, K.s, sd);
-      if ((e = hipGetLastError()) != hipSuccess) return e;
-    }
-    if ((e = launch_sh_gate(K, x, T, H, L.d.sh_gate_inp, sig)) != hipSuccess) return e;
-  }
-  return launch_combine(K, o, pair_of, idx, w, L.d.down_bias, T, k, H, osh, sig, y);
+  return launch_combine(K, f32_at(p.xo), go.pair_of, idx, w, L.d.down_bias, T, k, H, Ish ? f32_at(p.osh) : nullptr, sig, y);
 }
 
 }  // namespace mr

@@ -232,8 +232,10 @@ struct GroupedScratch {
   float* pair_w;      // [P] its routing weight
   int32_t* pair_of;   // [P] sorted index of (token, slot)
   int32_t* exp_off;   // [E+1] pair offset of each expert
-  int32_t* tile_off;  // [E+1] 16-pair tile offset of each expert
-  uint8_t* img_x;     // [T][H/32][128] x images
+  int32_t* tile_off;  // [E+1] pair tile offset of each expert
+  int32_t* tile_exp;  // expert of each pair tile
+  int32_t* hist;      // per-workgroup expert counts of the grouping (many pairs)
+  uint8_t* img_x;     // [T][H/32][128] x images (in obuf's memory)
   uint32_t* sc_x;     // [T][H/32]
   uint8_t* img_h;     // [P][I/32][128] h images
   uint32_t* sc_h;     // [P][I/32]
@@ -254,8 +256,20 @@ hipError_t launch_grouped(const Launch& K, const mr_layer& L, const float* x, ui
 // Pair grouping, grid size and the ascending-expert combine shared by the grouped paths
 // (mr_grouped.hip).
 unsigned grouped_grid(uint64_t items);
-hipError_t launch_group(const Launch& K, const int32_t* idx, const float* w, int P, int k, int E, int32_t* pair_tok,
-                        float* pair_w, int32_t* pair_of, int32_t* exp_off, int32_t* tile_off);
+struct GroupOut {
+  int32_t* pair_tok;  // [P] token of sorted pair p
+  float* pair_w;      // [P] its routing weight
+  int32_t* pair_of;   // [P] sorted index of (token, slot)
+  int32_t* exp_off;   // [E+1] pair offset of each expert
+  int32_t* tile_off;  // [E+1] pair tile offset of each expert
+  int32_t* tile_exp;  // [tile_off[E]] expert of each tile
+  int32_t* hist;      // scratch of group_hist_bytes
+};
+constexpr uint64_t kGroupTileMin = 16;  // the smallest pair tile of any grouped path
+inline uint64_t group_tiles_max(uint64_t P, uint64_t E, uint64_t tile) { return P / tile + std::min(P, E); }
+uint64_t group_hist_bytes(uint64_t P, uint64_t E);
+hipError_t launch_group(const Launch& K, const int32_t* idx, const float* w, int P, int k, int E, int tile,
+                        const GroupOut& o);
 hipError_t launch_combine(const Launch& K, const float* o, const int32_t* pair_of, const int32_t* idx, const float* w,
                           const float* down_b, uint32_t T, int k, int H, const float* o_sh, const float* sh_sig,
                           float* y);

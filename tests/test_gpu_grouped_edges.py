@@ -1,0 +1,91 @@
+"""The grouped multi-token kernels at the edges of their tiles: pair counts around the 16- and
+64-pair tiles and their 16-pair groups (all tokens on the same experts, so an expert's pairs are
+the tokens), means that select either pair tile, one and several super-blocks per row, row counts
+that fill half a tile, the shared expert's own width, and enough pairs for the grouping to take
+several workgroups. Reference: the per-token VALU path (f32 arithmetic, 3e-7 of the output), per
+token, max error over the token's largest output. Bar 2e-5 for Q4_K: the activations carry 22
+significant bits and sums are f32."""
+from dataclasses import replace
+
+import numpy as np
+import pytest
+
+import moe_rocm as M
+from moe_rocm import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+Q4 = W.LayerSpec(280, 0, W.GGML_Q4_K, 512, 256, 24, 3, W.ROUTE_NORM_TOPK, W.ACT_SILU, False, True)
+BAR = 2e-5
+
+
+def _batched(gpu_ctx, dl, x, kernel):
+    T, H = x.shape
+    dx, dy = gpu_ctx.to_device(x), gpu_ctx.alloc(T * H * 4)
+    gpu_ctx.set_option(M.OPT_DECODE_KERNEL, kernel)
+    try:
+        dl.layer.forward_batched(dx, T, dy)
+        gpu_ctx.sync()
+        return dy.download(np.float32).reshape(T, H)
+    finally:
+        gpu_ctx.set_option(M.OPT_DECODE_KERNEL, M.DECODE_AUTO)
+        dx.free(), dy.free()
+
+
+def _check(gpu_ctx, spec, T, one_route=False, bar=BAR):
+    host = W.host_layer(spec)
+    if one_route:  # the bias decides: every token takes the same top_k experts
+        host["router_b"] = (host["router_b"] + 1e3 * (np.arange(spec.n_experts) % 5 == 1)
+                            - np.arange(spec.n_experts)).astype(np.float32)
+    dl = W.DeviceLayer(gpu_ctx, spec, host=host)
+    try:
+        x = W.x_tokens(spec, T)
+        ref = _batched(gpu_ctx, dl, x, M.DECODE_VALU)
+        got = _batched(gpu_ctx, dl, x, M.DECODE_AUTO)
+        err = np.abs(got - ref).max(1) / np.abs(ref).max(1)
+        assert np.isfinite(got).all() and err.max() <= bar, (spec, T, float(err.max()), int(err.argmax()))
+    finally:
+        dl.close()
+
+
+@pytest.mark.parametrize("T", [1, 2, 15, 16, 17, 31, 33, 48, 49, 63, 64, 65, 129])
+def test_q4k_pairs_per_expert(gpu_ctx, T):
+    _check(gpu_ctx, Q4, T, one_route=True)
+
+
+@pytest.mark.parametrize("T", [64, 65])  # mean pairs per expert 8 and just above: the pair tile changes
+def test_q4k_pair_tile_rule(gpu_ctx, T):
+    _check(gpu_ctx, Q4, T)
+
+
+@pytest.mark.parametrize("H,I,sh", [(256, 256, 0), (768, 512, 256), (1280, 768, 1024), (2048, 256, 512)])
+@pytest.mark.parametrize("T", [5, 70])
+def test_q4k_widths_and_shared(gpu_ctx, H, I, sh, T):
+    _check(gpu_ctx, replace(Q4, hidden=H, inter=I, sh_inter=sh), T)
+
+
+@pytest.mark.parametrize("T", [2730, 2731, 5500])  # 8,190, 8,193 and 16,500 pairs: one, two and three workgroups
+def test_grouping_of_many_pairs(gpu_ctx, T):
+    _check(gpu_ctx, replace(Q4, hidden=256), T)
+
+
+def test_q4k_scales_zero_and_denormal_rows(gpu_ctx):
+    """Rows of zeros, of denormals, of 2^100 and of mixed magnitudes: the power-of-two row scale."""
+    spec = replace(Q4, hidden=512)
+    host = W.host_layer(spec)
+    host["router_w"] = np.zeros_like(host["router_w"])
+    dl = W.DeviceLayer(gpu_ctx, spec, host=host)
+    try:
+        x = W.x_tokens(spec, 20)
+        x[0] = 0.0
+        x[1] = 1e-40
+        x[2] *= np.float32(1e-30)
+        x[3] *= np.float32(2.0) ** 40
+        x[4, ::2] *= np.float32(1e-6)
+        ref = _batched(gpu_ctx, dl, x, M.DECODE_VALU)
+        got = _batched(gpu_ctx, dl, x, M.DECODE_AUTO)
+        assert np.array_equal(got[0], ref[0]) and np.abs(got[1]).max() <= 1e-30
+        for t in range(2, 20):
+            assert np.abs(got[t] - ref[t]).max() <= BAR * np.abs(ref[t]).max() + 1e-37, t
+    finally:
+        dl.close()
