@@ -45,15 +45,25 @@ __global__ __launch_bounds__(256) void k_router_logits(const float* __restrict__
   const float* xr = x + (size_t)t * H;
   const float* w = wr + (size_t)e * H;
   float acc = 0.f;
-  for (int c = lane * 4; c < H; c += 256) {
-    f32x4 a = *reinterpret_cast<const f32x4*>(xr + c);
-    f32x4 b = *reinterpret_cast<const f32x4*>(w + c);
-    acc = __builtin_fmaf(a.x, b.x, acc);
-    acc = __builtin_fmaf(a.y, b.y, acc);
-    acc = __builtin_fmaf(a.z, b.z, acc);
-    acc = __builtin_fmaf(a.w, b.w, acc);
+  // six steps' loads at once: latency bounds it (one step at a time: 7.3 us at H = 2880)
+  for (int c0 = lane * 4; c0 < H; c0 += 6 * 256) {
+    f32x4 a[6], b[6];
+#pragma unroll
+    for (int j = 0; j < 6; ++j) {
+      const int c = min(c0 + 256 * j, H - 4);
+      a[j] = *reinterpret_cast<const f32x4*>(xr + c);
+      b[j] = *reinterpret_cast<const f32x4*>(w + c);
+    }
+#pragma unroll
+    for (int j = 0; j < 6; ++j)
+      if (c0 + 256 * j < H) {
+        acc = __builtin_fmaf(a[j].x, b[j].x, acc);
+        acc = __builtin_fmaf(a[j].y, b[j].y, acc);
+        acc = __builtin_fmaf(a[j].z, b[j].z, acc);
+        acc = __builtin_fmaf(a[j].w, b[j].w, acc);
+      }
   }
-  acc = wave_sum(acc);
+  acc = wave_sum_fast(acc);
   if (lane == 0) {
     if (br) acc = acc + br[e];
     if (mask) acc = acc + mask[e];
@@ -72,53 +82,78 @@ __global__ __launch_bounds__(256) void k_router_logits(const float* __restrict__
 // their element j, so the four MFMAs cover the block's 16 elements; D[4g + r][i] is token
 // t0+4g+r, expert e0+i. Tokens past T and experts past E repeat the last row (not stored).
 // part: [nks][T][E]. H % 4 == 0 and ceil(H/16) <= nks * 16 * kRouterBlocks.
+// A workgroup takes TT x TE such tiles (TT token tiles, TE expert tiles) so that each loaded row
+// serves several: the loads, 16 rows to every 16 lanes, bound it (4,096 tokens x 128 experts x 2048:
+// 80 us with one tile each, 51 us with 2 x 2). A tile's sums are the same bits whatever TT and TE.
 constexpr int kRouterWaves = 16, kRouterBlocks = 6, kRouterMaxSplit = 4;
+template <int TT, int TE>
 __global__ __launch_bounds__(1024) void k_router_logits_mfma(const float* __restrict__ x,
                                                              const float* __restrict__ wr,
                                                              float* __restrict__ part, int T, int H, int E,
                                                              int nks) {
-  __shared__ f32x4 red[kRouterWaves][64];
+  __shared__ f32x4 red[TT * TE][kRouterWaves][64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int i = lane & 15, g = lane >> 4;
-  const int t0 = blockIdx.y * 16, e0 = blockIdx.x * 16;
+  const int t0 = blockIdx.y * (16 * TT), e0 = blockIdx.x * (16 * TE);
   const int nb = (H + 15) >> 4, per = (nb + nks - 1) / nks;
   const int kb0 = (int)blockIdx.z * per, kb1 = min(nb, kb0 + per);
-  const float* xr = x + (size_t)min(t0 + i, T - 1) * H + 4 * g;
-  const float* wrow = wr + (size_t)min(e0 + i, E - 1) * H + 4 * g;
+  const float* xr[TT];
+  const float* wrow[TE];
+#pragma unroll
+  for (int t = 0; t < TT; ++t) xr[t] = x + (size_t)min(t0 + 16 * t + i, T - 1) * H + 4 * g;
+#pragma unroll
+  for (int e = 0; e < TE; ++e) wrow[e] = wr + (size_t)min(e0 + 16 * e + i, E - 1) * H + 4 * g;
   const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-  f32x4 a[kRouterBlocks], w[kRouterBlocks];
+  f32x4 acc[TT][TE];
 #pragma unroll
-  for (int j = 0; j < kRouterBlocks; ++j) {
-    const int b = kb0 + wave + kRouterWaves * j;
-    const bool in = b < kb1 && 16 * b + 4 * g < H;
-    a[j] = in ? *reinterpret_cast<const f32x4*>(xr + 16 * b) : z;
-    w[j] = in ? *reinterpret_cast<const f32x4*>(wrow + 16 * b) : z;
-  }
-  f32x4 acc = z;
+  for (int t = 0; t < TT; ++t)
 #pragma unroll
-  for (int j = 0; j < kRouterBlocks; ++j) {
-    if (kb0 + wave + kRouterWaves * j < kb1) {  // wave-uniform
-      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j].x, w[j].x, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j].y, w[j].y, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j].z, w[j].z, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j].w, w[j].w, acc, 0, 0, 0);
+    for (int e = 0; e < TE; ++e) acc[t][e] = z;
+  constexpr int kAhead = TT * TE == 1 ? kRouterBlocks : kRouterBlocks / 2;  // blocks whose loads go out together
+#pragma unroll
+  for (int j0 = 0; j0 < kRouterBlocks; j0 += kAhead) {
+    f32x4 a[kAhead][TT], w[kAhead][TE];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      const int b = kb0 + wave + kRouterWaves * (j0 + j);
+      const bool in = b < kb1 && 16 * b + 4 * g < H;
+#pragma unroll
+      for (int t = 0; t < TT; ++t) a[j][t] = in ? *reinterpret_cast<const f32x4*>(xr[t] + 16 * b) : z;
+#pragma unroll
+      for (int e = 0; e < TE; ++e) w[j][e] = in ? *reinterpret_cast<const f32x4*>(wrow[e] + 16 * b) : z;
+    }
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      if (kb0 + wave + kRouterWaves * (j0 + j) < kb1) {  // wave-uniform
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+          for (int t = 0; t < TT; ++t)
+#pragma unroll
+            for (int e = 0; e < TE; ++e)
+              acc[t][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j][t][c], w[j][e][c], acc[t][e], 0, 0, 0);
+      }
     }
   }
-  red[wave][lane] = acc;
+#pragma unroll
+  for (int t = 0; t < TT; ++t)
+#pragma unroll
+    for (int e = 0; e < TE; ++e) red[t * TE + e][wave][lane] = acc[t][e];
   __syncthreads();
-  if (wave == 0) {
-    f32x4 s = red[0][lane];
+  if (wave < TT * TE) {
+    const f32x4(*r)[64] = red[wave];
+    f32x4 s = r[0][lane];
 #pragma unroll
     for (int q = 1; q < kRouterWaves; ++q) {
-      const f32x4 p = red[q][lane];
+      const f32x4 p = r[q][lane];
       s = f32x4{s[0] + p[0], s[1] + p[1], s[2] + p[2], s[3] + p[3]};
     }
-    const int e = e0 + i;
+    const int e = e0 + 16 * (wave % TE) + i;
     float* out = part + (size_t)blockIdx.z * T * E;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int t = t0 + 4 * g + r;
-      if (t < T && e < E) out[(size_t)t * E + e] = s[r];
+    for (int q = 0; q < 4; ++q) {
+      const int t = t0 + 16 * (wave / TE) + 4 * g + q;
+      if (t < T && e < E) out[(size_t)t * E + e] = s[q];
     }
   }
 }
@@ -284,8 +319,13 @@ hipError_t launch_router_topk(const Launch& K, const mr_layer& L, const float* x
   }
   {
     ProfScope ps(K, "router_logits");
-    hipLaunchKernelGGL(k_router_logits_mfma, dim3((L.E + 15) / 16, (T + 15) / 16, nks), dim3(64 * kRouterWaves), 0,
-                       K.s, x, L.d.router_w, part, (int)T, (int)L.H, (int)L.E, (int)nks);
+    // 2 x 2 tiles once the grid still spans the CUs with a quarter of the workgroups
+    if (tiles * nks >= 4 * 256)
+      hipLaunchKernelGGL((k_router_logits_mfma<2, 2>), dim3((L.E + 31) / 32, (T + 31) / 32, nks), dim3(64 * kRouterWaves),
+                         0, K.s, x, L.d.router_w, part, (int)T, (int)L.H, (int)L.E, (int)nks);
+    else
+      hipLaunchKernelGGL((k_router_logits_mfma<1, 1>), dim3((L.E + 15) / 16, (T + 15) / 16, nks), dim3(64 * kRouterWaves),
+                         0, K.s, x, L.d.router_w, part, (int)T, (int)L.H, (int)L.E, (int)nks);
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
