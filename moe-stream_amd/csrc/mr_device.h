@@ -87,12 +87,11 @@ __device__ __forceinline__ void mx_load_block(const uint8_t* p, uint32_t& scale,
 // Sum over one block of kvalue_j * x_j for the 32 elements of the block (GGUF
 // order: byte j low nibble -> element j, high nibble -> element j+16). The
 // caller multiplies by the block's half scale.
-__device__ __forceinline__ float mx_block_kdot(const uint32_t q[4], const float* xb) {
+__device__ __forceinline__ float mx_block_kdot(const uint32_t q[4], const f32x4 (&x)[8]) {
   float s0 = 0.f, s1 = 0.f;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const f32x4 xl = *reinterpret_cast<const f32x4*>(xb + 4 * i);
-    const f32x4 xh = *reinterpret_cast<const f32x4*>(xb + 16 + 4 * i);
+    const f32x4 xl = x[i], xh = x[4 + i];
     f32x2 v0 = MR_KV2(q[i], 0);
     f32x2 v1 = MR_KV2(q[i], 1);
     f32x2 v2 = MR_KV2(q[i], 2);
