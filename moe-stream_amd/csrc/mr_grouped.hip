@@ -5,17 +5,18 @@
 // the expert's tokens, gate/up/act/down, x routing weight, index_add back
 // (layer.rs:2148-2183; CPU: mxfp4_matmul per expert, layer.rs:1449-1514). Here:
 //   k_group       (token, slot) pairs grouped by expert; per-expert pair offsets and
-//                 32-pair tile offsets; pair index of every (token, slot).
+//                 pair tile offsets (tiles of 16, 32 or 64 pairs) and each tile's expert; pair
+//                 index of every (token, slot).
 //   k_split_rows  x rows -> e4m3 B images (terms 0-2 of the split of each 32-element block).
-//   k_grouped_gemm<true>   gate and up for one (expert, 128-row tile, 32-pair tile):
+//   k_grouped_gemm<true>   gate and up for one (expert, 128-row tile, pair tile):
 //                 A = native MXFP4 weight rows, B = the pairs' x images; epilogue
 //                 bias + activation x routing weight, split into the h images
 //                 [pair][I/32] (the split of k_split_rows).
-//   k_grouped_gemm<false>  down for one (expert, 256-row tile, 32-pair tile) on the
+//   k_grouped_gemm<false>  down for one (expert, 256-row tile, pair tile) on the
 //                 h images -> o [pair][H].
 //   k_combine     y[t] = sum over t's pairs in ascending expert order of
 //                 (o + w*b_down) (the order of layer.rs:1092-1106).
-// Every weight byte of an expert is read by the ceil(n_e/32) pair tiles of its
+// Every weight byte of an expert is read by the pair tiles of its
 // row tiles; work items are laid out so those repeats, and the repeats of the
 // pairs' activation images over row tiles, hit the same XCD's L2.
 #include "mr_device.h"
@@ -33,7 +34,6 @@ namespace mr {
 // compute and write (the images keep the 4-term layout; term 3 is left unwritten).
 constexpr int kGemmTerms = 3;
 
-constexpr int kPairTile = 32;   // pairs (tokens) per work item = 8 MFMA column groups x 4
 constexpr int kXcds = 8;        // MI355X accelerator complex dies (one L2 each)
 constexpr int kMaxSteps = 32;   // K steps (4 blocks) per row: K <= 4096
 
@@ -178,8 +178,9 @@ struct GroupedArgs {
   const float* pair_w;      // GATEUP: routing weight of pair p, or null (weight 1)
   const int32_t* exp_off;
   const int32_t* tile_off;
+  const int32_t* tile_exp;
   int single_p;  // > 0: one expert (e = 0) over pairs 0 .. single_p - 1 (the shared expert over
-                 // every token); exp_off and tile_off are not read
+                 // every token); exp_off, tile_off and tile_exp are not read
   float* out;        // [P][M] (down)
   uint8_t* himg;     // GATEUP: the down input images [P][M/32][kImgBytes]
   uint32_t* hsc;     // GATEUP: their scale words [P][M/32]
@@ -188,10 +189,10 @@ struct GroupedArgs {
   float alpha, limit;
 };
 
-// Grouped GEMM work item: (expert e, row tile, 32-pair tile); 4 waves. A wave owns kGT
+// Grouped GEMM work item: (expert e, row tile, tile of 16 kPG pairs); 4 waves. A wave owns kGT
 // 16-row A tiles (gate/up: 32 gate rows and the same 32 up rows, so that the activation and the
 // split of the down input image run in registers, 128 rows per item; down: 4 x 64 = 256 rows)
-// and the tile's 32 pairs as 2 groups of 16.
+// and the tile's pairs as kPG groups of 16.
 // The MFMAs take the first kGemmTerms = 3 e4m3 terms of the pairs' activation split (the
 // residual after three terms is below 2^-12 of each 32-element block's max, bf16 operands
 // hold 8 significant bits). A K step holds 4 weight blocks; MFMA m of the step takes term m of
@@ -200,18 +201,25 @@ struct GroupedArgs {
 // term's scale byte). A lane's A operand is then the same in the step's 3 MFMAs, so each A
 // window is read from LDS and aligned once per step, and D accumulates the term-summed dot
 // product of row x pair: no term columns to add afterwards, 16 pairs per MFMA, and a wave
-// keeps kGT x 2 accumulator tiles.
+// keeps kGT x kPG accumulator tiles.
 // K advances 4 blocks per step:
 //   A: each row's 68 bytes of a step as 6 aligned 16-byte pieces, lane-contiguous (a wave
 //      load covers ~11 rows' contiguous bytes; 20-byte windows loaded per lane straight
-//      from global cost 3x the L1 accesses), two steps ahead in registers, then written to
+//      from global cost 3x the L1 accesses), kAhead steps ahead in registers, then written to
 //      the wave's LDS slice, from which the 4 lanes of a row read the same block window;
-//   B: the step's 32 pairs x 4 blocks x the 96 bytes of terms 0-2 of their images (12 KB) and
-//      their scale words, one step ahead in registers (3 pieces per thread; the images are L2
-//      hits), then written to a double-buffered LDS stage shared by the 4 waves. (Direct global->LDS loads would save the registers, but
-//      the compiler then waits for all of them before any LDS read, which serialises the
-//      prefetch.) 16-byte part q of (pair pr, block b) sits in slot b_slot(pr, b, q),
-//      so the 16 lanes of a read (16 pairs, one part) hit 16 different bank groups.
+//   B: the step's pairs x 4 blocks x the 96 bytes of terms 0-2 of their images (6 KB per pair
+//      group) and their scale words, one step ahead in registers (the images are L2 hits), then
+//      written to a double-buffered LDS stage shared by the 4 waves. (Direct global->LDS loads
+//      would save the registers, but the compiler then waits for all of them before any LDS
+//      read, which serialises the prefetch.)
+// What bounds it: the per-step chain (stage written, barrier, LDS reads, alignment, MFMAs) at two
+// or three waves per SIMD; a step on 64 pairs issues 48 MFMAs per wave for one such chain, on 32
+// pairs 24. 64 pairs fit the registers since the A loads take a scalar base and 32-bit offsets
+// (64-bit addresses with 64-bit limits: 239 VGPRs at 32 pairs, now 194) and the B operands are
+// read per pair group. 2,039 tokens of 4 in 32 experts of 2880 x 2880: 610 + 308 us for the two
+// launches in 32-pair tiles with the expert searched in the tile offsets, now 524 + 269 us (512
+// TFLOP/s of layer arithmetic, 3 times that issued). 4 tokens: 46 + 28 us, now 40 + 25 us in
+// 16-pair tiles.
 constexpr int kGW = 4;               // waves per work item
 #ifndef MR_GROUPED_GT_GU
 #define MR_GROUPED_GT_GU 4
@@ -222,8 +230,6 @@ constexpr int kGW = 4;               // waves per work item
 // 16-row A tiles per wave (gate/up, down) and the rows of a matrix per work item
 template <bool GATEUP> constexpr int kGTof = GATEUP ? MR_GROUPED_GT_GU : MR_GROUPED_GT_DN;
 template <bool GATEUP> constexpr int kRowsOf = (GATEUP ? kGW / 2 : kGW) * kGTof<GATEUP> * 16;
-constexpr int kPG = kPairTile / 16;  // 16-pair MFMA column groups
-constexpr int kBStep = kPairTile * 4 * kImgBytes;  // B bytes per K step
 constexpr int kAPR = 6;                            // A pieces per row and step: 68 bytes at any offset
 #ifndef MR_GROUPED_AROW
 #define MR_GROUPED_AROW 104
@@ -231,18 +237,16 @@ constexpr int kAPR = 6;                            // A pieces per row and step:
 constexpr int kARow = MR_GROUPED_AROW;  // LDS bytes per A row: 26 dwords, so 16 rows fall in 16 different banks
 static_assert(kARow % 4 == 0 && kARow >= 6 * 16, "an A row holds a step's 6 pieces, dword-aligned");
 constexpr int kBBuf = 2;                           // B stages in LDS
-static_assert(kBStep == 4 * kGW * 64 * 16, "room for four 16-byte pieces per thread per step");
-constexpr int kBPieces = 3;  // 16-byte B pieces loaded per thread and step (terms 0-2)
-static_assert(kPairTile * 4 * 6 == kBPieces * kGW * 64, "the pieces of terms 0-2 fill the threads");
-static_assert(kPairTile * 4 == 2 * 64, "scale words: one per lane of waves 0-1");
 static_assert(kTerms == 4, "images of 4 terms (8 parts of 16 bytes per block); the GEMMs read terms 0-2");
+constexpr int kBParts = 4 * 6;  // 16-byte parts of a pair per K step: 4 blocks x terms 0-2
 
-// LDS slot of 16-byte part q of (pair pr, block b) in a B stage: the 16 pairs that one read
-// instruction's lanes take (one part each) land in 16 different 16-byte bank groups.
-__device__ __forceinline__ int b_slot(int pr, int b, int q) { return pr * 32 + (b ^ ((pr >> 3) & 1)) * 8 + (q ^ (pr & 7)); }
-
-template <bool GATEUP>
-__global__ __launch_bounds__(256, 2) void k_grouped_gemm(GroupedArgs a) {
+template <bool GATEUP, int kPG>
+__global__ __launch_bounds__(256, kPG == 1 ? 3 : 2) void k_grouped_gemm(GroupedArgs a) {
+  constexpr int kPairTile = 16 * kPG;
+  // LDS slot (16 bytes) of part q (0 .. 5) of (pair pr, block b) in a B stage: (6 b + q) kBRow + pr
+  constexpr int kBRow = kPairTile + 1;
+  constexpr int kBStep = kBParts * kBRow * 16;  // bytes of a stage
+  constexpr int kBPieces = (kPairTile * kBParts + 255) / 256;  // 16-byte pieces loaded per thread and step
   __shared__ __align__(16) uint8_t bst[kBBuf][kBStep];
   __shared__ __align__(16) uint32_t bsc[kBBuf][kPairTile * 4];
   constexpr int kGT = kGTof<GATEUP>;               // 16-row A tiles per wave
@@ -267,12 +271,8 @@ __global__ __launch_bounds__(256, 2) void k_grouped_gemm(GroupedArgs a) {
   const int loc = blockIdx.x / kXcds;
   const int w = (blockIdx.x % kXcds) * per_xcd + loc;
   if (loc >= per_xcd || w >= n_work) return;  // uniform: no work item for this workgroup
-  int lo = 0, hi = single ? 1 : a.E;  // expert: n_rt * tile_off[e] <= w < n_rt * tile_off[e+1]
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (n_rt * a.tile_off[mid] <= w) lo = mid; else hi = mid;
-  }
-  const int e = lo;
+  // expert: n_rt * tile_off[e] <= w < n_rt * tile_off[e+1], so pair tile w / n_rt is one of its own
+  const int e = single ? 0 : a.tile_exp[w / n_rt];
   const int e_beg = single ? 0 : a.exp_off[e], e_end = single ? a.single_p : a.exp_off[e + 1];
   const int nt_e = single ? n_tiles : a.tile_off[e + 1] - a.tile_off[e];
   const int wl = w - (single ? 0 : n_rt * a.tile_off[e]);
@@ -309,34 +309,43 @@ __global__ __launch_bounds__(256, 2) void k_grouped_gemm(GroupedArgs a) {
   for (int mt = 0; mt < 2; ++mt)
     lead0[mt] = (uint32_t)(reinterpret_cast<uintptr_t>(Wm[mt]) + (uintptr_t)min(wrow0 + i, a.M - 1) * rb) & 15u;
   // A piece slots of this lane: slot k*64 + lane = (tile, row, piece) of the wave's rows
-  const uint8_t* aps[kAK];
-  int apc[kAK], aslot[kAK];
+  // A load's matrix is the same in all lanes: its 16-byte aligned base stays in scalar registers
+  // and a lane keeps 32-bit offsets (a matrix holds at most 4,096 rows of 2,176 bytes): that of
+  // its piece at step 0, unaligned, and that of the row's last piece.
+  static_assert((16 * kAPR * kTR) % 64 == 0, "a load's slots lie in one matrix");
+  const uint8_t* abase[2];
+#pragma unroll
+  for (int mt = 0; mt < 2; ++mt)
+    abase[mt] = reinterpret_cast<const uint8_t*>(reinterpret_cast<uintptr_t>(Wm[mt]) & ~(uintptr_t)15);
+  uint32_t aoff[kAK], alast[kAK];
+  int aslot[kAK];
 #pragma unroll
   for (int k = 0; k < kAK; ++k) {
     const int sl = min(k * 64 + lane, kASlots - 1);
     const int tt = sl / (16 * kAPR), rr = (sl / kAPR) % 16;
-    apc[k] = sl % kAPR;
-    aps[k] = Wm[tt / kTR] + (uint64_t)min(wrow0 + 16 * (tt % kTR) + rr, a.M - 1) * rb;
-    aslot[k] = (tt * 16 + rr) * kARow + apc[k] * 16;
+    const uint32_t row = ((uint32_t)reinterpret_cast<uintptr_t>(Wm[k * 64 / (16 * kAPR * kTR)]) & 15u) +
+                         (uint32_t)min(wrow0 + 16 * (tt % kTR) + rr, a.M - 1) * (uint32_t)rb;
+    aoff[k] = row + 16u * (uint32_t)(sl % kAPR);
+    alast[k] = (row + (uint32_t)rb - 1u) & ~15u;
+    aslot[k] = (tt * 16 + rr) * kARow + (sl % kAPR) * 16;
   }
 
-  // B pieces of this thread: the step's 32 pairs x 4 blocks x the 6 16-byte parts of terms
-  // 0-2 (term 3 is not used) are 768 pieces, 3 per thread: piece j*256 + tid = (pair, block,
-  // part) in that order, so consecutive lanes read consecutive parts of a block
+  // B pieces of this thread: piece j*256 + tid = (pair, block, part) in that order, so
+  // consecutive lanes read consecutive parts of a block (threads past the last piece repeat it)
   const uint8_t* bsrc[kBPieces];
   int bslot[kBPieces], bblk[kBPieces];
 #pragma unroll
   for (int j = 0; j < kBPieces; ++j) {
-    const int q = j * 256 + tid, part = q % 6, blk = (q / 6) & 3, pr = q / 24;
-    bslot[j] = b_slot(pr, blk, part);
+    const int q = min(j * 256 + tid, kPairTile * kBParts - 1), part = q % 6, blk = (q / 6) & 3, pr = q / 24;
+    bslot[j] = (blk * 6 + part) * kBRow + pr;
     bblk[j] = blk;
     const int p = p0 + min(pr, np - 1);
     const int r = a.pair_tok ? a.pair_tok[p] : p;
     bsrc[j] = a.img + (size_t)r * nbK * kImgBytes + part * 16;
   }
-  const uint32_t* ssrc;  // scale word tid (waves 0-1): pair tid/4, block tid%4
+  const uint32_t* ssrc;  // scale word tid (the first 4 kPairTile threads): pair tid/4, block tid%4
   {
-    const int p = p0 + min((tid & 127) >> 2, np - 1);
+    const int p = p0 + min(tid >> 2, np - 1);
     const int r = a.pair_tok ? a.pair_tok[p] : p;
     ssrc = a.isc + (size_t)r * nbK;
   }
@@ -355,15 +364,13 @@ __global__ __launch_bounds__(256, 2) void k_grouped_gemm(GroupedArgs a) {
   auto store_b = [&](const BRegs& br, int buf) {
 #pragma unroll
     for (int j = 0; j < kBPieces; ++j) *reinterpret_cast<i32x4*>(&bst[buf][bslot[j] * 16]) = br.v[j];
-    if (wave < 2) bsc[buf][tid] = br.sc;
+    if (wave < kPG) bsc[buf][tid] = br.sc;  // 4 kPairTile words: kPG waves
   };
   auto load_a = [&](int st, i32x4 (&apv)[kAK]) {  // pieces past the row end read its last piece
 #pragma unroll
     for (int k = 0; k < kAK; ++k) {
-      const uintptr_t first = (reinterpret_cast<uintptr_t>(aps[k]) + (uintptr_t)(68 * st)) & ~(uintptr_t)15;
-      const uintptr_t last = (reinterpret_cast<uintptr_t>(aps[k]) + (uintptr_t)(17 * nbK) - 1) & ~(uintptr_t)15;
-      const uintptr_t src = min(first + 16 * (uintptr_t)apc[k], last);
-      apv[k] = *(const __attribute__((address_space(1))) i32x4*)src;
+      const uint32_t src = min((aoff[k] + 68u * (uint32_t)st) & ~15u, alast[k]);
+      apv[k] = *(const __attribute__((address_space(1))) i32x4*)(abase[k * 64 / (16 * kAPR * kTR)] + src);
     }
   };
   auto store_a = [&](const i32x4 (&apv)[kAK]) {  // slots past kASlots are not stored
@@ -385,20 +392,22 @@ __global__ __launch_bounds__(256, 2) void k_grouped_gemm(GroupedArgs a) {
   // (pair i of the group, K group g): its A operand is weight block g of the step in all three
   // MFMAs; its B bytes 0-15 are K [16g, 16g+16), half g%2 of K block g/2, and bytes 16-31 half
   // g%2 of K block 2 + g/2, i.e. part 2m + g%2 of (pair i, block g/2) and of (pair i, block
-  // 2 + g/2), which b_slot places 16 slots (256 bytes) further; its B scale byte is (pair i,
-  // block g, term m) at 16i + 4g + m. Pairs of the two groups differ by 16 (the same swizzle;
-  // scale bytes +256). brdp holds the slot of MFMA m's first part in bits 10m .. 10m + 9.
-  uint32_t brdp = 0u;
-#pragma unroll
-  for (int mm = 0; mm < 3; ++mm) brdp |= (uint32_t)b_slot(i, g >> 1, 2 * mm + (g & 1)) << (10 * mm);
+  // 2 + g/2), 12 kBRow slots further; its B scale byte is (pair i, block g, term m) at 16i + 4g + m.
+  // A stage's slots are part-major: the 16 lanes of a read take 16 neighbouring slots, and the
+  // odd row length spreads the consecutive parts that a wave writes over the banks.
+  const int brd0 = (((g >> 1) * 6 + (g & 1)) * kBRow + i) * 16;
   const int sc_lane = i * 16 + 4 * g;
-  auto brd = [&](int mm) { return (int)(__builtin_amdgcn_ubfe(brdp, 10u * (uint32_t)mm, 10u) * 16u); };
 
-  i32x4 apA[kAK], apB[kAK];
+  // A loads run kAhead steps ahead: two (a register set for each parity) where a step is short;
+  // one step of 4 pair groups covers them, and the second set would spill. Measured (the whole
+  // call, us, 32 experts of 2880 x 2880, 4 per token), two against one: 128 tokens on 2 groups
+  // 192 / 197, 32 tokens on 1 group 156 / 160, 2039 tokens on 4 groups 787 / 780.
+  constexpr int kAhead = kPG == 4 ? 1 : 2;
+  i32x4 apv[kAhead][kAK];
   BRegs bR;
   load_b(0, bR);
-  load_a(0, apA);
-  load_a(min(1, S - 1), apB);
+#pragma unroll
+  for (int d = 0; d < kAhead; ++d) load_a(min(d, S - 1), apv[d]);
 
   f32x4 acc[kGT][kPG];
 #pragma unroll
@@ -419,28 +428,25 @@ __global__ __launch_bounds__(256, 2) void k_grouped_gemm(GroupedArgs a) {
     store_b(bR, buf);  // buffer st % 2 was last read in step st-2, before the previous barrier
     __syncthreads();   // step st's B stage is complete
     load_b(min(st + 1, S - 1), bR);
-    load_a(min(st + 2, S - 1), cur);
+    load_a(min(st + kAhead, S - 1), cur);
     const uint8_t* bb_base = &bst[buf][0];
     const uint8_t* sc_base = reinterpret_cast<const uint8_t*>(&bsc[buf][0]);
     uint32_t wo[2];  // per matrix: block g's scale byte in the row's LDS slice (68 st = 4 st mod 16)
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt) wo[mt] = ((lead0[mt] + 4u * (uint32_t)st) & 15u) + 17u * (uint32_t)g;
-    // B operands of MFMA mm for the 2 pair groups, read one MFMA ahead; the A operands (this
-    // lane's block g of each tile's row i) once per step for all three MFMAs. A block past the
-    // row end (read inside the LDS stage) gets zero codes, so it adds nothing.
+    // B operands of (term mm, pair group pg), read two ahead of their MFMAs; the A operands (this
+    // lane's block g of each tile's row i) once per step for all MFMAs. A block past the row end
+    // (read inside the LDS stage) gets zero codes, so it adds nothing.
     struct BOps {
-      i32x4 b[kPG][2];
-      int sb[kPG];
+      i32x4 b[2];
+      int sb;
     };
-    auto read_b = [&](int mm, BOps& o) {
-      const int off = brd(mm);
-#pragma unroll
-      for (int pg = 0; pg < kPG; ++pg) {
-        const uint8_t* bp = bb_base + pg * 16 * 32 * 16 + off;  // pairs 16 further: same swizzle
-        o.b[pg][0] = *reinterpret_cast<const i32x4*>(bp);
-        o.b[pg][1] = *reinterpret_cast<const i32x4*>(bp + 256);
-        o.sb[pg] = (int)sc_base[sc_lane + mm + pg * 256];
-      }
+    auto read_b = [&](int n, BOps& o) {
+      const int mm = n / kPG, pg = n % kPG;
+      const uint8_t* bp = bb_base + brd0 + (2 * mm * kBRow + 16 * pg) * 16;
+      o.b[0] = *reinterpret_cast<const i32x4*>(bp);
+      o.b[1] = *reinterpret_cast<const i32x4*>(bp + 12 * kBRow * 16);
+      o.sb = (int)sc_base[sc_lane + mm + pg * 256];
     };
     RawBlk r[kGT];
 #pragma unroll
@@ -448,9 +454,9 @@ __global__ __launch_bounds__(256, 2) void k_grouped_gemm(GroupedArgs a) {
       const uint32_t* wp = reinterpret_cast<const uint32_t*>(&ast[wave][(tt * 16 + i) * kARow + (wo[tt / kTR] & ~3u)]);
       r[tt].d[0] = wp[0], r[tt].d[1] = wp[1], r[tt].d[2] = wp[2], r[tt].d[3] = wp[3], r[tt].d[4] = wp[4];
     }
-    BOps o0, o1;
-    read_b(0, o0);
-    read_b(1, o1);
+    BOps o[3];
+    read_b(0, o[0]);
+    read_b(1, o[1]);
     const bool valid = !kPart || 4 * st + g < nbK;
     AOp ao[kGT];
     int sa[kGT];
@@ -467,34 +473,30 @@ __global__ __launch_bounds__(256, 2) void k_grouped_gemm(GroupedArgs a) {
       }
       sa[tt] = valid ? (int)((r[tt].d[0] >> (8u * w3)) & 0xFFu) : 127;
     }
-    auto run_b = [&](const BOps& o) {
 #pragma unroll
-      for (int pg = 0; pg < kPG; ++pg) {
-        if (pg < npg) {
-          const i32x8 B = {o.b[pg][0][0], o.b[pg][0][1], o.b[pg][0][2], o.b[pg][0][3],
-                           o.b[pg][1][0], o.b[pg][1][1], o.b[pg][1][2], o.b[pg][1][3]};
+    for (int n = 0; n < kGemmTerms * kPG; ++n) {
+      if (n + 2 < kGemmTerms * kPG) read_b(n + 2, o[(n + 2) % 3]);
+      const int pg = n % kPG;
+      if (pg < npg) {
+        const BOps& c = o[n % 3];
+        const i32x8 B = {c.b[0][0], c.b[0][1], c.b[0][2], c.b[0][3], c.b[1][0], c.b[1][1], c.b[1][2], c.b[1][3]};
 #pragma unroll
-          for (int tt = 0; tt < kGT; ++tt)  // tiles past M repeat row M-1; their rows are not stored
-            acc[tt][pg] = mfma_op(ao[tt], sa[tt], B, o.sb[pg], acc[tt][pg]);
-        }
+        for (int tt = 0; tt < kGT; ++tt)  // tiles past M repeat row M-1; their rows are not stored
+          acc[tt][pg] = mfma_op(ao[tt], sa[tt], B, c.sb, acc[tt][pg]);
       }
-    };
-    run_b(o0);
-    read_b(2, o0);
-    run_b(o1);
-    run_b(o0);
+    }
   };
   // Steps 0 .. nbK/4 - 1 hold only blocks inside the row; the one or two steps after the loop
   // (the last one possibly partial) run the checked variant.
   const int s_full = nbK >> 2;
   int st = 0;
   for (; st + 1 < s_full; st += 2) {
-    step(st, apA, std::false_type{});
-    step(st + 1, apB, std::false_type{});
+    step(st, apv[0], std::false_type{});
+    step(st + 1, apv[kAhead - 1], std::false_type{});
   }
   if (st < S) {
-    step(st, apA, std::true_type{});
-    if (st + 1 < S) step(st + 1, apB, std::true_type{});
+    step(st, apv[0], std::true_type{});
+    if (st + 1 < S) step(st + 1, apv[kAhead - 1], std::true_type{});
   }
 
   // Epilogue: acc[tt][pg][r] of lane (i, g) is row wrow0 + 16 tt + 4g + r x pair 16 pg + i.
@@ -518,6 +520,7 @@ __global__ __launch_bounds__(256, 2) void k_grouped_gemm(GroupedArgs a) {
   const int nbM = a.M >> 5;
 #pragma unroll
   for (int pg = 0; pg < kPG; ++pg) {
+    if (pg >= npg) break;  // uniform
     const int pl = pg * 16 + i;
     const float pw = bias_s[2 * kRows + min(pl, kPairTile - 1)];
     float hv[2][4];  // [tile][r]: row 16 tile + 4g + r
@@ -720,14 +723,44 @@ hipError_t launch_combine(const Launch& K, const float* o, const int32_t* pair_o
 // (workgroup b takes item (b mod 8) * ceil(n_work / 8) + b / 8).
 unsigned grouped_grid(uint64_t items) { return (unsigned)((items + kXcds - 1) / kXcds * kXcds); }
 
+// One grouped GEMM launch over at most `tiles` pair tiles of 16 kPG pairs.
+template <bool GATEUP>
+static hipError_t launch_gemm(const Launch& K, const GroupedArgs& a, int pg, uint64_t tiles) {
+  constexpr int rows = kRowsOf<GATEUP>;
+  const dim3 grid(grouped_grid((uint64_t)((a.M + rows - 1) / rows) * tiles)), block(kGW * 64);
+  if (pg == 4)
+    hipLaunchKernelGGL((k_grouped_gemm<GATEUP, 4>), grid, block, 0, K.s, a);
+  else if (pg == 2)
+    hipLaunchKernelGGL((k_grouped_gemm<GATEUP, 2>), grid, block, 0, K.s, a);
+  else
+    hipLaunchKernelGGL((k_grouped_gemm<GATEUP, 1>), grid, block, 0, K.s, a);
+  return hipGetLastError();
+}
+
+// 16-pair groups per work item, for `pairs` pairs over `experts` experts with `rows` gate rows.
+// More groups reuse a step's weight windows and their alignment for more MFMAs; fewer waste less
+// on part-filled tiles and leave room for three workgroups per CU. The lines lie at a mean of 8
+// and 64 pairs per expert (whole call, us, 32 experts of 2880 x 2880, 1 / 2 / 4 groups: mean 4
+// 156 / 172 / 185; 8 162 / 176 / 195; 16 203 / 192 / 205; 64 370 / 308 / 298 and, with popularity
+// ~ rank^-1.1, 401 / 324 / 323 with a slower down launch; 128 620 / 492 / 447; 255 1166 / 911 / 780). Few work items take fewer groups, so that the CUs are not left idle: below two items per
+// CU 4 groups lose to 2 (16 experts of 1600 x 1504, 500 tokens of 4, 372 items: 113 / 109 us),
+// below one 2 lose to 1 (8 experts of 1024 x 512, 40 tokens of 4: 69 / 59 us).
+static int pair_groups(uint64_t pairs, uint64_t experts, int rows) {
+  int pg = pairs > 64 * experts ? 4 : pairs > 8 * experts ? 2 : 1;
+  const uint64_t n_rt = (uint64_t)((rows + kRowsOf<true> - 1) / kRowsOf<true>);
+  while (pg > 1 && std::max(pairs / (16 * pg), std::min(pairs, experts)) * n_rt < 128u * pg) pg >>= 1;
+  return pg;
+}
+
 hipError_t launch_grouped(const Launch& K, const mr_layer& L, const float* x, uint32_t T, const int32_t* idx,
                           const float* w, float* y, const GroupedScratch& gs) {
   const int k = (int)L.d.top_k, E = (int)L.E, H = (int)L.H, I = (int)L.I;
   const int P = (int)T * k;
-  const int max_tiles = (P + kPairTile - 1) / kPairTile + E;
+  const int pg = pair_groups((uint64_t)P, (uint64_t)E, I), tile = 16 * pg;
+  const uint64_t max_tiles = group_tiles_max((uint64_t)P, (uint64_t)E, (uint64_t)tile);
   hipError_t e;
   const GroupOut go{gs.pair_tok, gs.pair_w, gs.pair_of, gs.exp_off, gs.tile_off, gs.tile_exp, gs.hist};
-  if ((e = launch_group(K, idx, w, P, k, E, kPairTile, go)) != hipSuccess) return e;
+  if ((e = launch_group(K, idx, w, P, k, E, tile, go)) != hipSuccess) return e;
   {
     ProfScope ps(K, "split_x");
     hipLaunchKernelGGL(k_split_rows, dim3((unsigned)((H / 32 + 31) / 32), std::min<uint32_t>(T, 65535u)), dim3(256), 0,
@@ -738,21 +771,18 @@ hipError_t launch_grouped(const Launch& K, const mr_layer& L, const float* x, ui
   a.w0 = expert_loc(L.d.gate), a.w1 = expert_loc(L.d.up);
   a.b0 = L.d.gate_bias, a.b1 = L.d.up_bias;
   a.img = gs.img_x, a.isc = gs.sc_x, a.pair_tok = gs.pair_tok, a.pair_w = gs.pair_w;
-  a.exp_off = gs.exp_off, a.tile_off = gs.tile_off, a.himg = gs.img_h, a.hsc = gs.sc_h;
+  a.exp_off = gs.exp_off, a.tile_off = gs.tile_off, a.tile_exp = gs.tile_exp, a.himg = gs.img_h, a.hsc = gs.sc_h;
   a.M = I, a.K = H, a.E = E;
   a.act = (int)L.d.act, a.alpha = L.d.alpha, a.limit = L.d.limit;
   {
     ProfScope ps(K, "grouped_gateup");
-    constexpr int rows = kRowsOf<true>;
-    hipLaunchKernelGGL(k_grouped_gemm<true>, dim3(grouped_grid((uint64_t)((I + rows - 1) / rows) * max_tiles)), dim3(kGW * 64), 0,
-                       K.s, a);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if ((e = launch_gemm<true>(K, a, pg, max_tiles)) != hipSuccess) return e;
   }
   // The shared expert (layer.rs:1898-1953): one group of every token on the same x images,
   // weight 1 and SiLU (the routed experts' activation does not apply), its down outputs
   // [T][H], then sigmoid(x . gate_inp) per token, which the combine applies after the routed
   // sum.
-  const int Ish = L.d.sh_gate ? (int)L.Ish : 0, tiles = ((int)T + kPairTile - 1) / kPairTile;
+  const int Ish = L.d.sh_gate ? (int)L.Ish : 0, pgs = pair_groups(T, 1, Ish), tiles = ((int)T + 16 * pgs - 1) / (16 * pgs);
   if (Ish) {
     GroupedArgs sg{};
     sg.w0 = expert_loc(L.d.sh_gate), sg.w1 = expert_loc(L.d.sh_up);
@@ -761,23 +791,17 @@ hipError_t launch_grouped(const Launch& K, const mr_layer& L, const float* x, ui
     sg.M = Ish, sg.K = H, sg.E = 1, sg.act = MR_ACT_SILU;
     {
       ProfScope ps(K, "grouped_shared_gateup");
-      constexpr int rows = kRowsOf<true>;
-      hipLaunchKernelGGL(k_grouped_gemm<true>, dim3(grouped_grid((uint64_t)((Ish + rows - 1) / rows) * tiles)),
-                         dim3(kGW * 64), 0, K.s, sg);
-      if ((e = hipGetLastError()) != hipSuccess) return e;
+      if ((e = launch_gemm<true>(K, sg, pgs, tiles)) != hipSuccess) return e;
     }
   }
   GroupedArgs d{};
   d.w0 = expert_loc(L.d.down);
   d.img = gs.img_h, d.isc = gs.sc_h, d.pair_tok = nullptr, d.pair_w = gs.pair_w;
-  d.exp_off = gs.exp_off, d.tile_off = gs.tile_off, d.out = gs.obuf;
+  d.exp_off = gs.exp_off, d.tile_off = gs.tile_off, d.tile_exp = gs.tile_exp, d.out = gs.obuf;
   d.M = H, d.K = I, d.E = E;
   {
     ProfScope ps(K, "grouped_down");
-    constexpr int rows = kRowsOf<false>;
-    hipLaunchKernelGGL(k_grouped_gemm<false>, dim3(grouped_grid((uint64_t)((H + rows - 1) / rows) * max_tiles)), dim3(kGW * 64), 0,
-                       K.s, d);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if ((e = launch_gemm<false>(K, d, pg, max_tiles)) != hipSuccess) return e;
   }
   if (!Ish) return launch_combine(K, gs.obuf, gs.pair_of, idx, w, L.d.down_bias, T, k, H, nullptr, nullptr, y);
   GroupedArgs sd{};
@@ -786,10 +810,7 @@ hipError_t launch_grouped(const Launch& K, const mr_layer& L, const float* x, ui
   sd.M = H, sd.K = Ish, sd.E = 1;
   {
     ProfScope ps(K, "grouped_shared_down");
-    constexpr int rows = kRowsOf<false>;
-    hipLaunchKernelGGL(k_grouped_gemm<false>, dim3(grouped_grid((uint64_t)((H + rows - 1) / rows) * tiles)),
-                       dim3(kGW * 64), 0, K.s, sd);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if ((e = launch_gemm<false>(K, sd, pgs, tiles)) != hipSuccess) return e;
   }
   if ((e = launch_sh_gate(K, x, T, H, L.d.sh_gate_inp, gs.sig)) != hipSuccess) return e;
   return launch_combine(K, gs.obuf, gs.pair_of, idx, w, L.d.down_bias, T, k, H, gs.osh, gs.sig, y);

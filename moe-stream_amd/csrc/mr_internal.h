@@ -273,7 +273,7 @@ hipError_t launch_group(const Launch& K, const int32_t* idx, const float* w, int
 hipError_t launch_combine(const Launch& K, const float* o, const int32_t* pair_of, const int32_t* idx, const float* w,
                           const float* down_b, uint32_t T, int k, int H, const float* o_sh, const float* sh_sig,
                           float* y);
-// Grouped multi-token Q4_K path on the int8 MFMA (mr_grouped_q4k.hip); scratch: one block of
+// Grouped multi-token Q4_K path on the f16 MFMA (mr_grouped_q4k.hip); scratch: one block of
 // grouped_q4k_scratch_bytes.
 bool grouped_q4k_supported(const mr_layer& L);
 uint64_t grouped_q4k_scratch_bytes(uint64_t T, uint64_t k, uint64_t E, uint64_t I, uint64_t H, uint64_t Ish);

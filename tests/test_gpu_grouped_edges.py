@@ -1,4 +1,4 @@
-"""The grouped multi-token kernels at the edges of their tiles: pair counts around the 16- and
+"""The grouped multi-token kernels at the edges of their tiles: pair counts around the 16-, 32- and
 64-pair tiles and their 16-pair groups (all tokens on the same experts, so an expert's pairs are
 the tokens), means that select either pair tile, one and several super-blocks per row, row counts
 that fill half a tile, the shared expert's own width, and enough pairs for the grouping to take
@@ -62,6 +62,28 @@ def test_q4k_pair_tile_rule(gpu_ctx, T):
 @pytest.mark.parametrize("T", [5, 70])
 def test_q4k_widths_and_shared(gpu_ctx, H, I, sh, T):
     _check(gpu_ctx, replace(Q4, hidden=H, inter=I, sh_inter=sh), T)
+
+
+# MXFP4: the activations carry three 8-bit float terms; what they leave is below 2^-12 of a block's
+# largest value in each of the two products.
+MX = W.LayerSpec(281, 0, W.GGML_MXFP4, 288, 2080, 24, 3, W.ROUTE_SOFTMAX_AFTER_TOPK, W.ACT_SWIGLU_OAI, True, True)
+MX_BAR = 2.0 ** -11
+
+
+# 17 row tiles of the 2,080 gate rows (the last of 32 rows), 9 blocks per row of 288; every token on the
+# same three experts. 16-pair tiles up to 64 tokens (a mean of 8 pairs per expert), then 32-pair tiles,
+# 64-pair tiles from about 680 tokens on (512 work items); the counts leave the last tile around each
+# edge of its 16-pair groups.
+@pytest.mark.parametrize("T", [1, 2, 15, 16, 17, 33, 64, 65, 80, 81, 96, 97, 256, 683, 704, 705, 720, 721, 735, 737,
+                               753])
+def test_mxfp4_pairs_per_expert(gpu_ctx, T):
+    _check(gpu_ctx, MX, T, one_route=True, bar=MX_BAR)
+
+
+@pytest.mark.parametrize("H,I,sh", [(32, 32, 0), (160, 96, 0), (1056, 288, 2080), (2880, 160, 64)])
+@pytest.mark.parametrize("T", [5, 150, 1100])  # 1,100 tokens x 17 row tiles: the shared expert in 32-pair tiles
+def test_mxfp4_widths_and_shared(gpu_ctx, H, I, sh, T):
+    _check(gpu_ctx, replace(MX, hidden=H, inter=I, sh_inter=sh, sh_type=W.GGML_MXFP4), T, bar=MX_BAR)
 
 
 @pytest.mark.parametrize("T", [2730, 2731, 5500])  # 8,190, 8,193 and 16,500 pairs: one, two and three workgroups
