@@ -800,8 +800,9 @@ int mr_moe_forward_residual(mr_ctx* c, const mr_layer* L, const float* h, const 
 }
 
 // Routing and experts for T tokens (scratch already sized for T): the grouped GEMM path of the
-// layer's type, else the per-token VALU kernels.
-static hipError_t batched_core(mr_ctx* c, const mr_layer* L, const float* x, uint32_t T, float* y) {
+// layer's type, else the per-token VALU kernels. resid: [T, H] added to the result, or null.
+static hipError_t batched_core(mr_ctx* c, const mr_layer* L, const float* x, uint32_t T, float* y,
+                               const float* resid = nullptr) {
   mr::Scratch& s = c->scratch;
   float* lg = L->logits_out ? L->logits_out : s.logits;  // T <= logits_cap checked by the caller
   hipError_t e = mr::launch_router_topk(c->launch(), *L, x, T, lg, s.rpart, s.idx, s.w);
@@ -809,11 +810,13 @@ static hipError_t batched_core(mr_ctx* c, const mr_layer* L, const float* x, uin
     const Batched kind = batched_kind(c, *L);
     if (kind == Batched::grouped_mx)
       e = mr::launch_grouped(c->launch(), *L, x, T, s.idx, s.w, y,
-                             mr::grouped_scratch(s, s.cap_tokens, s.cap_k, s.cap_e, s.cap_i, s.cap_h, s.cap_ish));
+                             mr::grouped_scratch(s, s.cap_tokens, s.cap_k, s.cap_e, s.cap_i, s.cap_h, s.cap_ish), resid);
     else if (kind == Batched::grouped_q4k)
-      e = mr::launch_grouped_q4k(c->launch(), *L, x, T, s.idx, s.w, y, s.grouped);
-    else
-      e = mr::launch_experts_valu(c->launch(), *L, x, T, s.idx, s.w, s.act, s.act_sh, y);
+      e = mr::launch_grouped_q4k(c->launch(), *L, x, T, s.idx, s.w, y, s.grouped, resid);
+    else {
+      e = mr::launch_experts_valu(c->launch(), *L, x, T, s.idx, s.w, s.act, s.act_sh, resid ? s.ytmp : y);
+      if (e == hipSuccess && resid) e = mr::launch_residual_add(c->launch(), resid, s.ytmp, (uint64_t)T * L->H, y);
+    }
   }
   return e;
 }
@@ -849,8 +852,7 @@ int mr_moe_forward_batched_residual(mr_ctx* c, const mr_layer* L, const float* h
   if ((rc = bind(c)) || (rc = ensure_scratch(c, L, T))) return rc;
   mr::Scratch& s = c->scratch;
   hipError_t e = mr::launch_rms_norm(c->launch(), h, norm_w, eps, T, L->H, s.xn);
-  if (e == hipSuccess) e = batched_core(c, L, s.xn, T, s.ytmp);
-  if (e == hipSuccess) e = mr::launch_residual_add(c->launch(), h, s.ytmp, (uint64_t)T * L->H, h_out);
+  if (e == hipSuccess) e = batched_core(c, L, s.xn, T, h_out, h);
   return e == hipSuccess ? MR_OK : hip_fail(c, e, "batched moe residual launch");
 }
 

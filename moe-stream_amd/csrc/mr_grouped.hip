@@ -551,7 +551,9 @@ __global__ __launch_bounds__(256, kPG == 1 ? 3 : 2) void k_grouped_gemm(GroupedA
 // ---- combine -----------------------------------------------------------------------------
 // y[t][row] = sum over t's pairs in ascending pair index (= ascending expert) of
 // o[pair][row] + w * b_down[e][row], then + sig[t] * o_sh[t][row] when a shared expert ran
-// (layer.rs:1935-1951). One thread per (token, 4 rows) on a (row groups, tokens) grid (tokens
+// (layer.rs:1935-1951); with a residual input, y = resid + that (layer.rs:462-473; resid may be y:
+// a thread reads what it overwrites). Added here it costs one read of h; as a launch of its own it
+// read the sum back and wrote it again (2,039 tokens of 2880: 16 us after this kernel's 20; 4: 4.7). One thread per (token, 4 rows) on a (row groups, tokens) grid (tokens
 // past gridDim.y loop); the token's (at most KM) pair indices stay in registers and are taken
 // smallest first, and all of a thread's loads issue before the sums. H % 4 == 0.
 template <int KM>
@@ -559,7 +561,7 @@ __global__ __launch_bounds__(256) void k_combine(const float* __restrict__ o, co
                                                  const int32_t* __restrict__ idx, const float* __restrict__ w,
                                                  const float* __restrict__ down_b, int T, int k, int H,
                                                  const float* __restrict__ o_sh, const float* __restrict__ sh_sig,
-                                                 float* __restrict__ y) {
+                                                 const float* resid, float* y) {
   const int row = (blockIdx.x * 256 + threadIdx.x) * 4;
   if (row >= H) return;
   for (int t = blockIdx.y; t < T; t += gridDim.y) {
@@ -585,6 +587,8 @@ __global__ __launch_bounds__(256) void k_combine(const float* __restrict__ o, co
         }
       }
     }
+    f32x4 hv = {0.f, 0.f, 0.f, 0.f};
+    if (resid) hv = *reinterpret_cast<const f32x4*>(resid + (size_t)t * H + row);
     f32x4 sv = {0.f, 0.f, 0.f, 0.f};
     float sg = 0.f;
     if (o_sh) {
@@ -606,6 +610,9 @@ __global__ __launch_bounds__(256) void k_combine(const float* __restrict__ o, co
     if (o_sh)
 #pragma unroll
       for (int c = 0; c < 4; ++c) acc[c] = acc[c] + sg * sv[c];
+    if (resid)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[c] = hv[c] + acc[c];
     *reinterpret_cast<f32x4*>(y + (size_t)t * H + row) = acc;
   }
 }
@@ -703,18 +710,18 @@ hipError_t launch_group(const Launch& K, const int32_t* idx, const float* w, int
 
 hipError_t launch_combine(const Launch& K, const float* o, const int32_t* pair_of, const int32_t* idx, const float* w,
                           const float* down_b, uint32_t T, int k, int H, const float* o_sh, const float* sh_sig,
-                          float* y) {
+                          const float* resid, float* y) {
   ProfScope ps(K, "combine");
   const dim3 grid((unsigned)((H / 4 + 255) / 256), std::min<uint32_t>(T, 65535u));
   if (k <= 4)
     hipLaunchKernelGGL(k_combine<4>, grid, dim3(256), 0, K.s, o, pair_of, idx, w, down_b, (int)T, k, H, o_sh, sh_sig,
-                       y);
+                       resid, y);
   else if (k <= 8)
     hipLaunchKernelGGL(k_combine<8>, grid, dim3(256), 0, K.s, o, pair_of, idx, w, down_b, (int)T, k, H, o_sh, sh_sig,
-                       y);
+                       resid, y);
   else
     hipLaunchKernelGGL(k_combine<16>, grid, dim3(256), 0, K.s, o, pair_of, idx, w, down_b, (int)T, k, H, o_sh,
-                       sh_sig, y);
+                       sh_sig, resid, y);
   return hipGetLastError();
 }
 
@@ -753,7 +760,7 @@ static int pair_groups(uint64_t pairs, uint64_t experts, int rows) {
 }
 
 hipError_t launch_grouped(const Launch& K, const mr_layer& L, const float* x, uint32_t T, const int32_t* idx,
-                          const float* w, float* y, const GroupedScratch& gs) {
+                          const float* w, float* y, const GroupedScratch& gs, const float* resid) {
   const int k = (int)L.d.top_k, E = (int)L.E, H = (int)L.H, I = (int)L.I;
   const int P = (int)T * k;
   const int pg = pair_groups((uint64_t)P, (uint64_t)E, I), tile = 16 * pg;
@@ -803,7 +810,7 @@ hipError_t launch_grouped(const Launch& K, const mr_layer& L, const float* x, ui
     ProfScope ps(K, "grouped_down");
     if ((e = launch_gemm<false>(K, d, pg, max_tiles)) != hipSuccess) return e;
   }
-  if (!Ish) return launch_combine(K, gs.obuf, gs.pair_of, idx, w, L.d.down_bias, T, k, H, nullptr, nullptr, y);
+  if (!Ish) return launch_combine(K, gs.obuf, gs.pair_of, idx, w, L.d.down_bias, T, k, H, nullptr, nullptr, resid, y);
   GroupedArgs sd{};
   sd.w0 = expert_loc(L.d.sh_down);
   sd.img = gs.img_hsh, sd.isc = gs.sc_hsh, sd.single_p = (int)T, sd.out = gs.osh;
@@ -813,7 +820,7 @@ hipError_t launch_grouped(const Launch& K, const mr_layer& L, const float* x, ui
     if ((e = launch_gemm<false>(K, sd, pgs, tiles)) != hipSuccess) return e;
   }
   if ((e = launch_sh_gate(K, x, T, H, L.d.sh_gate_inp, gs.sig)) != hipSuccess) return e;
-  return launch_combine(K, gs.obuf, gs.pair_of, idx, w, L.d.down_bias, T, k, H, gs.osh, gs.sig, y);
+  return launch_combine(K, gs.obuf, gs.pair_of, idx, w, L.d.down_bias, T, k, H, gs.osh, gs.sig, resid, y);
 }
 
 }  // namespace mr

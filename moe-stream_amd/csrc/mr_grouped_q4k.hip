@@ -631,7 +631,7 @@ bool grouped_q4k_supported(const mr_layer& L) {
 }
 
 hipError_t launch_grouped_q4k(const Launch& K, const mr_layer& L, const float* x, uint32_t T, const int32_t* idx,
-                              const float* w, float* y, void* scratch) {
+                              const float* w, float* y, void* scratch, const float* resid) {
   const int k = (int)L.d.top_k, E = (int)L.E, H = (int)L.H, I = (int)L.I, Ish = L.d.sh_gate ? (int)L.Ish : 0;
   // The kernels address the images of a call's rows within kPast bytes: more tokens than that
   // holds run in parts (a token's result depends on that token alone).
@@ -639,7 +639,8 @@ hipError_t launch_grouped_q4k(const Launch& K, const mr_layer& L, const float* x
   if (T > T_max) {
     for (uint32_t t0 = 0; t0 < T; t0 += T_max) {
       const hipError_t e = launch_grouped_q4k(K, L, x + (size_t)t0 * H, std::min(T_max, T - t0), idx + (size_t)t0 * k,
-                                              w + (size_t)t0 * k, y + (size_t)t0 * H, scratch);
+                                              w + (size_t)t0 * k, y + (size_t)t0 * H, scratch,
+                                              resid ? resid + (size_t)t0 * H : nullptr);
       if (e != hipSuccess) return e;
     }
     return hipSuccess;
@@ -707,7 +708,8 @@ hipError_t launch_grouped_q4k(const Launch& K, const mr_layer& L, const float* x
       hipLaunchKernelGGL((k_grouped_q4k<false, 4>), grid, dim3(64 * q4_waves(false, 4)), 0, K.s, d);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
-  return launch_combine(K, f32_at(p.xo), go.pair_of, idx, w, L.d.down_bias, T, k, H, Ish ? f32_at(p.osh) : nullptr, sig, y);
+  return launch_combine(K, f32_at(p.xo), go.pair_of, idx, w, L.d.down_bias, T, k, H, Ish ? f32_at(p.osh) : nullptr, sig,
+                        resid, y);
 }
 
 }  // namespace mr

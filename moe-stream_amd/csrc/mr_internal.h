@@ -251,8 +251,9 @@ uint64_t grouped_scratch_bytes(uint64_t T, uint64_t k, uint64_t E, uint64_t I, u
 // sigmoid(x_t . gate_inp) per token t, or 1 without gate_inp (mr_grouped_q4k.hip)
 hipError_t launch_sh_gate(const Launch& K, const float* x, uint32_t T, int H, const float* gate_inp, float* sig);
 bool grouped_supported(const mr_layer& L);
+// resid: a [T][H] input added to the result, y = resid + moe (y may be resid), or null.
 hipError_t launch_grouped(const Launch& K, const mr_layer& L, const float* x, uint32_t T, const int32_t* idx,
-                          const float* w, float* y, const GroupedScratch& gs);
+                          const float* w, float* y, const GroupedScratch& gs, const float* resid = nullptr);
 // Pair grouping, grid size and the ascending-expert combine shared by the grouped paths
 // (mr_grouped.hip).
 unsigned grouped_grid(uint64_t items);
@@ -272,13 +273,13 @@ hipError_t launch_group(const Launch& K, const int32_t* idx, const float* w, int
                         const GroupOut& o);
 hipError_t launch_combine(const Launch& K, const float* o, const int32_t* pair_of, const int32_t* idx, const float* w,
                           const float* down_b, uint32_t T, int k, int H, const float* o_sh, const float* sh_sig,
-                          float* y);
+                          const float* resid, float* y);
 // Grouped multi-token Q4_K path on the f16 MFMA (mr_grouped_q4k.hip); scratch: one block of
 // grouped_q4k_scratch_bytes.
 bool grouped_q4k_supported(const mr_layer& L);
 uint64_t grouped_q4k_scratch_bytes(uint64_t T, uint64_t k, uint64_t E, uint64_t I, uint64_t H, uint64_t Ish);
 hipError_t launch_grouped_q4k(const Launch& K, const mr_layer& L, const float* x, uint32_t T, const int32_t* idx,
-                              const float* w, float* y, void* scratch);
+                              const float* w, float* y, void* scratch, const float* resid = nullptr);
 bool fused_q4k_supported(const mr_layer& L, int n_cu);
 bool fused_q4k_resident(const mr_layer& L, int n_cu);
 hipError_t launch_fused_q4k(const Launch& K, const mr_layer& L, const float* x, float* y, uint32_t* err,

@@ -86,6 +86,40 @@ def test_mxfp4_widths_and_shared(gpu_ctx, H, I, sh, T):
     _check(gpu_ctx, replace(MX, hidden=H, inter=I, sh_inter=sh, sh_type=W.GGML_MXFP4), T, bar=MX_BAR)
 
 
+@pytest.mark.parametrize("spec", [replace(MX, hidden=1056, inter=288), replace(Q4, hidden=768, sh_inter=512),
+                                  replace(MX, hidden=160, inter=96, sh_inter=64, sh_type=W.GGML_MXFP4)])
+@pytest.mark.parametrize("kernel", [M.DECODE_AUTO, M.DECODE_VALU])
+@pytest.mark.parametrize("T", [2, 33])
+def test_residual_added_in_the_combine(gpu_ctx, spec, kernel, T):
+    """h + moe(norm(h)) is the plain call's result on the normed rows plus h, and the same bits
+    into another buffer and in place."""
+    dl = W.DeviceLayer(gpu_ctx, spec, host=W.host_layer(spec))
+    h = W.x_tokens(spec, T) * np.float32(2.0) ** -3
+    one = np.ones(spec.hidden, np.float32)
+    zero = np.zeros_like(h)
+    dh, dn, dy, dz = (gpu_ctx.to_device(v) for v in (h, one, zero, zero))
+    gpu_ctx.set_option(M.OPT_DECODE_KERNEL, kernel)
+    try:
+        dl.layer.forward_batched_residual(dh, T, dn, 1e-5, dy)
+        dl.layer.forward_batched_residual(dh, T, dn, 1e-5, dh)
+        gpu_ctx.sync()
+        out, in_place = dy.download(np.float32), dh.download(np.float32)
+        assert np.array_equal(out, in_place)
+        normed = (h * (np.float32(1) / np.sqrt((h.astype(np.float64) ** 2).mean(1, keepdims=True) + 1e-5))).astype(np.float32)
+        dx = gpu_ctx.to_device(normed)
+        dl.layer.forward_batched(dx, T, dz)
+        gpu_ctx.sync()
+        want = h + dz.download(np.float32).reshape(h.shape)
+        # the norm's own rounding (a few 2^-24 of its sum of squares) passes through the layer
+        assert np.abs(out.reshape(h.shape) - want).max() <= MX_BAR * np.abs(want).max()
+        dx.free()
+    finally:
+        gpu_ctx.set_option(M.OPT_DECODE_KERNEL, M.DECODE_AUTO)
+        for b in (dh, dn, dy, dz):
+            b.free()
+        dl.close()
+
+
 @pytest.mark.parametrize("T", [2730, 2731, 5500])  # 8,190, 8,193 and 16,500 pairs: one, two and three workgroups
 def test_grouping_of_many_pairs(gpu_ctx, T):
     _check(gpu_ctx, replace(Q4, hidden=256), T)
