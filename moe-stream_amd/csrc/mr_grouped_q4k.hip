@@ -8,10 +8,12 @@
 //                      the f16 nearest to the rest, p a power of two per row: 22 significant
 //                      bits) plus the f32 sum of every 32-element sub-block as three f16 terms;
 //                      with a shared expert also its sigmoid gate of the row.
-//   k_grouped_q4k<1>   gate and up for one (expert, 256 rows, pair tile); epilogue bias +
-//                      activation x routing weight, split into the down input images (a tile's
-//                      256 rows are one super-block of the down input, with its own p).
-//   k_grouped_q4k<0>   down for one (expert, 256 rows, pair tile) -> o [pair][H].
+//   k_grouped_q4k<1>   gate and up for one (expert, 64, 128 or 256 rows, pair tile); epilogue bias +
+//                      activation x routing weight -> h, in f32 in the down input images' place or,
+//                      where the item's 256 rows are one super-block of the down input, split into
+//                      its image, with its own p.
+//   k_split_h          h in f32 -> the down input images, in place.
+//   k_grouped_q4k<0>   down for one (expert, 128 or 256 rows, pair tile) -> o [pair][H].
 //   k_combine          (mr_grouped.hip) the pairs of a token in ascending expert order, then the
 //                      shared expert scaled by its sigmoid gate (layer.rs:1092-1106, 1935-1951).
 // The shared expert is one more group (every token, weight 1, SiLU) of the same two launches.
@@ -79,6 +81,25 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const uint8_t* p, ui
 }
 
 // ---- activation rows -> images ----------------------------------------------------------------
+// Image of a super-block: lane l holds elements 4l .. 4l+3, v. Element 4l + c: h = l >> 5, g / 2 =
+// l >> 4 & 1, hl = l >> 3 & 1, g % 2 = l >> 2 & 1, u = l >> 1 & 1, bytes 4 (l & 1) + c, i.e. halves
+// 4 (l & 1) + {0, 2, 1, 3}.
+__device__ __forceinline__ void split_sb(f32x4 v, float p, int lane, uint8_t* dst) {
+  const int at = (4 * (lane >> 5) + (lane & 2) + ((lane >> 3) & 1)) * 128 +
+                 (2 * ((lane >> 4) & 1) + ((lane >> 2) & 1)) * 16 + (lane & 1) * 8;
+  uint32_t h[4], l[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) split2(v[c] * p, h[c], l[c]);
+  *reinterpret_cast<uint2*>(dst + at) = make_uint2(h[0] | h[2] << 16, h[1] | h[3] << 16);
+  *reinterpret_cast<uint2*>(dst + at + 64) = make_uint2(l[0] | l[2] << 16, l[1] | l[3] << 16);
+  float ps = (v.x + v.y) + (v.z + v.w);  // sub-block sum over the 8 lanes 8j .. 8j+7
+  ps += dpp_f<kDppXor1>(ps);
+  ps += dpp_f<kDppXor2>(ps);
+  ps = add_xor4(ps);
+  const int t = lane & 7, j = lane >> 3;
+  if (t < 4) *reinterpret_cast<uint16_t*>(dst + 1024 + t * 16 + kQPerm[j] * 2) = (uint16_t)sum_term(ps * p, t);
+}
+
 // One workgroup per row, its waves over the row's super-blocks in turn (lane l: elements 4l ..
 // 4l+3), twice: the row's largest magnitude, then the split (the second read hits L1). sig: the
 // shared expert's gate sigmoid(x . gate_inp) of the row, 1 without gate_inp (layer.rs:1935-1951).
@@ -111,25 +132,24 @@ __global__ __launch_bounds__(256) void k_split_f16(const float* __restrict__ src
     pinv_out[r] = pinv;
     if (sig) sig[r] = gi ? sigmoidf_((red[4] + red[5]) + (red[6] + red[7])) : 1.0f;
   }
-  // element 4l + c of the super-block: h = l >> 5, g / 2 = l >> 4 & 1, hl = l >> 3 & 1, g % 2 =
-  // l >> 2 & 1, u = l >> 1 & 1, bytes 4 (l & 1) + c, i.e. halves 4 (l & 1) + {0, 2, 1, 3}
-  const int at = (4 * (lane >> 5) + (lane & 2) + ((lane >> 3) & 1)) * 128 +
-                 (2 * ((lane >> 4) & 1) + ((lane >> 2) & 1)) * 16 + (lane & 1) * 8;
-  for (int sb = wave; sb < nsb; sb += 4) {
-    const f32x4 v = *reinterpret_cast<const f32x4*>(row + sb * 256 + 4 * lane);
-    uint8_t* dst = img + ((size_t)r * nsb + sb) * kQImgSb;
-    uint32_t h[4], l[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) split2(v[c] * p, h[c], l[c]);
-    *reinterpret_cast<uint2*>(dst + at) = make_uint2(h[0] | h[2] << 16, h[1] | h[3] << 16);
-    *reinterpret_cast<uint2*>(dst + at + 64) = make_uint2(l[0] | l[2] << 16, l[1] | l[3] << 16);
-    float ps = (v.x + v.y) + (v.z + v.w);  // sub-block sum over the 8 lanes 8j .. 8j+7
-    ps += dpp_f<kDppXor1>(ps);
-    ps += dpp_f<kDppXor2>(ps);
-    ps = add_xor4(ps);
-    const int t = lane & 7, j = lane >> 3;
-    if (t < 4) *reinterpret_cast<uint16_t*>(dst + 1024 + t * 16 + kQPerm[j] * 2) = (uint16_t)sum_term(ps * p, t);
-  }
+  for (int sb = wave; sb < nsb; sb += 4)
+    split_sb(*reinterpret_cast<const f32x4*>(row + sb * 256 + 4 * lane), p, lane, img + ((size_t)r * nsb + sb) * kQImgSb);
+}
+
+// h, one super-block in f32 at the start of each image's place -> the images: a wave per super-block,
+// which it holds in registers before it writes. The routed pairs' n0 super-blocks, then the shared
+// expert's n1 (a launch of their own: 4.7 us).
+__global__ __launch_bounds__(256) void k_split_h(uint8_t* img0, float* pinv0, int64_t n0, uint8_t* img1, float* pinv1,
+                                                 int64_t n1) {
+  const int lane = threadIdx.x & 63;
+  const int64_t b = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (b >= n0 + n1) return;
+  uint8_t* dst = b < n0 ? img0 + (size_t)b * kQImgSb : img1 + (size_t)(b - n0) * kQImgSb;
+  const f32x4 v = *reinterpret_cast<const f32x4*>(dst + 16 * lane);
+  float p, pinv;
+  pow2_scale(wave_max(fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)))), p, pinv);
+  if (lane == 0) *(b < n0 ? pinv0 + b : pinv1 + (b - n0)) = pinv;
+  split_sb(v, p, lane, dst);
 }
 
 // ---- shared-expert gate: sigmoid(x . gate_inp) per token (layer.rs:1935-1951) -------------------
@@ -153,7 +173,7 @@ struct GQ4Group {
   const float* b1;     // up bias
   const uint8_t* img;  // images [rows][K/256]
   const float* pinv;   // their 1/p: [rows] (GATEUP), [rows][K/256] (down)
-  uint8_t* himg;       // GATEUP: the down input images [pairs][M/256]
+  uint8_t* himg;       // GATEUP: the down input images [pairs][M/256], or h in f32 (256 floats) at each one's start
   float* hpinv;        // and their 1/p
   float* out;          // down: [pairs][M]
   int M, K, act;
@@ -169,11 +189,12 @@ struct GQ4Args {
   float alpha, limit;
 };
 
-// Work item: (expert e, 256 rows of each matrix, tile of 16 PG pairs). Gate/up: 16 waves, wave w
-// rows 16 w .. 16 w + 15 of the gate and of the up matrix, so that a lane holds both values of a
-// (row, pair) and a down input super-block (256 rows of h) forms inside one item; down: 8 waves of
-// 32 rows (PG = 1: two workgroups on a CU) or 4 of 64 rows (PG = 4: 323 instead of 348 us at the
-// size below, as its accumulators fit there). The activations are the MFMA's A operand (rows:
+// Work item: (expert e, rows of each matrix, tile of 16 PG pairs), NW waves. Gate/up: wave w rows
+// 16 w .. 16 w + 15 of the gate and of the up matrix, so that a lane holds both values of a
+// (row, pair). NW = 16, 256 rows: a down input super-block forms inside one item, which splits it;
+// NW = 8 or 4: h goes through memory, for k_split_h. Down: 4 waves of 32 rows (PG = 1) or of 64 (PG = 4:
+// 323 us at the size below, with 8 of 32 rows 348, as its accumulators fit there). Which of them runs:
+// see launch_grouped_q4k. The activations are the MFMA's A operand (rows:
 // pairs), the weights its B operand (columns: weight rows): lane (i, g) = lane % 16, lane / 16
 // holds weight row i of every tile, and of D weight row i for pairs 4g .. 4g+3 of each pair group.
 //   A wave's weights come in halves of a super-block, 64 bytes per row, one or two halves ahead in
@@ -191,14 +212,16 @@ struct GQ4Args {
 // on long batches: 128 experts of 768 x 2048, 32,768 pairs: gate/up 1.00 -> 0.60 ms and down
 // 0.49 -> 0.32 ms against the int8 MFMA with its scale products on the accumulators per sub-block.
 // Few pairs: the same unpacking against the weight stream (512 experts of 512 x 2048, 3,840
-// pairs: gate/up 300 -> 225 us, 2.7 TB/s; 128 pairs of 128 experts of 768 x 2048: 78 -> 48 us).
-// 16-row tiles per wave (see the kernel), and its waves
+// pairs: gate/up 300 -> 191 us, 3.1 TB/s; 128 pairs of 128 experts of 768 x 2048: 78 -> 37 us).
+// 16-row tiles per wave (see the kernel), and the rows of a matrix per work item
 constexpr int q4_tiles(bool gateup, int pg) { return gateup || pg == 1 ? 2 : 4; }
-constexpr int q4_waves(bool gateup, int pg) { return (gateup ? 32 : 16) / q4_tiles(gateup, pg); }
+constexpr int q4_rows(bool gateup, int pg, int waves) { return 16 * q4_tiles(gateup, pg) / (gateup ? 2 : 1) * waves; }
 
-template <bool GATEUP, int PG>
-__global__ __launch_bounds__(64 * q4_waves(GATEUP, PG), q4_tiles(GATEUP, PG) == 4 ? 2 : 4) void k_grouped_q4k(GQ4Args a) {
-  constexpr int NT = q4_tiles(GATEUP, PG), NW = q4_waves(GATEUP, PG);
+template <bool GATEUP, int PG, int NW>
+__global__ __launch_bounds__(64 * NW, q4_tiles(GATEUP, PG) == 4 ? 2 : 4) void k_grouped_q4k(GQ4Args a) {
+  constexpr int NT = q4_tiles(GATEUP, PG), kRows = q4_rows(GATEUP, PG, NW);
+  static_assert(256 % kRows == 0, "row counts are multiples of 256");
+  constexpr bool kSplit = GATEUP && kRows == 256;  // the epilogue writes images
   constexpr int kTM = GATEUP ? NT / 2 : NT;  // tiles of one matrix per wave
   constexpr int kPF = PG == 1 ? 2 : 1;       // half super-blocks of weights in flight
   constexpr int kKS = PG == 1 ? 8 : 2;       // K steps per stage
@@ -207,20 +230,20 @@ __global__ __launch_bounds__(64 * q4_waves(GATEUP, PG), q4_tiles(GATEUP, PG) == 
   constexpr int kStage = kKS * 2 * PG * 1024;
   constexpr int kPairs = 16 * PG;
   constexpr int kEpRow = kQImgSb + 16;  // epilogue: bytes between the images of two pairs
-  constexpr int kEp = GATEUP ? kPairs * kEpRow : 0;
+  constexpr int kEp = kSplit ? kPairs * kEpRow : 0;
   __shared__ __align__(16) uint8_t lds[kEp > 2 * kStage ? kEp : 2 * kStage];
   __shared__ __align__(16) uint8_t xst[2][PG == 1 ? 16 : PG * 1024];  // sub-block sums, operand order (PG = 1: in registers)
   __shared__ __align__(16) uint8_t ast[NW][NT * 1024];  // half a super-block of the wave's rows: [tile][row][64 bytes]
   __shared__ __align__(16) uint8_t hst[NW][NT * 256];   // and their headers: [tile][row][16 bytes]
   __shared__ __align__(16) float pst[2][kPairs];       // down: 1/p of (pair, super-block); gate/up: [0] of the pair
   __shared__ __align__(16) float pw[kPairs];           // GATEUP: routing weights
-  __shared__ __align__(16) float wred[GATEUP ? NW : 1][kPairs], wsum[GATEUP && NT == 2 ? NW : 1][kPairs];
+  __shared__ __align__(16) float wred[kSplit ? NW : 1][kPairs], wsum[kSplit && NT == 2 ? NW : 1][kPairs];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int i = lane & 15, g = lane >> 4;
   const int n_sh_t = (a.sh_T + kPairs - 1) / kPairs;
-  const int n_rt_s = (a.s.M + 255) >> 8, n_rt_r = (a.r.M + 255) >> 8;
+  const int n_rt_s = a.s.M / kRows, n_rt_r = a.r.M / kRows;
   const int n_sh = a.sh_T ? n_rt_s * n_sh_t : 0;
   const int n_work = n_sh + n_rt_r * a.tile_off[a.E];
   const int per_xcd = (n_work + kQXcds - 1) / kQXcds;
@@ -246,7 +269,7 @@ __global__ __launch_bounds__(64 * q4_waves(GATEUP, PG), q4_tiles(GATEUP, PG) == 
   const uint32_t rb = (uint32_t)nsb * 144u;
   // tile t of this wave: GATEUP: gate (t < kTM) or up rows wrow0 + 16 (t % kTM) .. ; down: rows wrow0
   // + 16 t .. . M % 256 == 0.
-  const int wrow0 = rt * 256 + wave * (16 * kTM);
+  const int wrow0 = rt * kRows + wave * (16 * kTM);
   // Buffer loads: one lane offset for all tiles, the tile and super-block in the scalar offset.
   const __amdgpu_buffer_rsrc_t wb0 = buffer_of(expert_at(q.w0, e), (uint32_t)M * rb);
   const __amdgpu_buffer_rsrc_t wb1 = GATEUP ? buffer_of(expert_at(q.w1, e), (uint32_t)M * rb) : wb0;
@@ -279,7 +302,7 @@ __global__ __launch_bounds__(64 * q4_waves(GATEUP, PG), q4_tiles(GATEUP, PG) == 
       const int pg = (wave * kPW + c) % PG;
       brow[c] = pg < NPG ? (uint32_t)row_of(16 * pg + lr) * ib + 16 * lp : (uint32_t)kPast;
     }
-    // (K step, term) of the pieces: kPW <= PG pieces share one, or each has its own (PG = 1)
+    // (K step, term) of the pieces: those of one share it
     auto bkt = [&](int c) { return (uint32_t)((wave * kPW + c) / PG) * 64u; };
     // the sub-block sums: PG = 1: the lane's own operand; else waves 0 .. NPG-1 bring those of
     // pair group `wave`
@@ -481,11 +504,8 @@ __global__ __launch_bounds__(64 * q4_waves(GATEUP, PG), q4_tiles(GATEUP, PG) == 
       }
     } else {
       // h = act(gate + b_g, up + b_u) x routing weight in registers (this lane: rows 16 t + i of
-      // the wave's, pairs 4g + r of each group), then the item's 256 rows of a pair, one
-      // super-block, are split. Largest magnitudes and sums go over the
-      // 16 lanes of a row group, the magnitudes over the waves through LDS; the halves are put
-      // in place in LDS and leave as whole 16-byte pieces.
-      float hv[kTM][NPG][4], hsum[NPG][4];
+      // the wave's, pairs 4g + r of each group).
+      float hv[kTM][NPG][4];
 #pragma unroll
       for (int t = 0; t < kTM; ++t) {
         const int row = wrow0 + 16 * t + i;
@@ -501,64 +521,84 @@ __global__ __launch_bounds__(64 * q4_waves(GATEUP, PG), q4_tiles(GATEUP, PG) == 
           }
         }
       }
+      if constexpr (!kSplit) {
 #pragma unroll
-      for (int pg = 0; pg < NPG; ++pg)
+        for (int t = 0; t < kTM; ++t) {
+          const int row = wrow0 + 16 * t + i;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          float m = fmaxf(fabsf(hv[0][pg][r]), fabsf(hv[kTM - 1][pg][r])), s = kTM == 2 ? hv[0][pg][r] + hv[kTM - 1][pg][r] : hv[0][pg][r];
-          m = fmaxf(m, dpp_f<kDppXor1>(m)), s += dpp_f<kDppXor1>(s);
-          m = fmaxf(m, dpp_f<kDppXor2>(m)), s += dpp_f<kDppXor2>(s);
-          m = fmaxf(m, dpp_f<kDppHMirror>(m)), s += dpp_f<kDppHMirror>(s);
-          m = fmaxf(m, dpp_f<kDppMirror>(m)), s += dpp_f<kDppMirror>(s);
-          hsum[pg][r] = s;
-          if (i == 0) {
-            wred[wave][16 * pg + 4 * g + r] = m;
-            if (NT == 2) wsum[wave][16 * pg + 4 * g + r] = s;  // half a sub-block
+          for (int pg = 0; pg < NPG; ++pg)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const int pl = 16 * pg + 4 * g + r;
+              if (pl < np)
+                reinterpret_cast<float*>(q.himg + ((size_t)(p0 + pl) * (M >> 8) + (row >> 8)) * kQImgSb)[row & 255] =
+                    hv[t][pg][r];
+            }
+        }
+      } else {
+        // The item's 256 rows of a pair, one super-block, are split. Largest magnitudes and sums go
+        // over the 16 lanes of a row group, the magnitudes over the waves through LDS; the halves
+        // are put in place in LDS and leave as whole 16-byte pieces.
+        float hsum[NPG][4];
+#pragma unroll
+        for (int pg = 0; pg < NPG; ++pg)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            float m = fmaxf(fabsf(hv[0][pg][r]), fabsf(hv[kTM - 1][pg][r])), s = kTM == 2 ? hv[0][pg][r] + hv[kTM - 1][pg][r] : hv[0][pg][r];
+            m = fmaxf(m, dpp_f<kDppXor1>(m)), s += dpp_f<kDppXor1>(s);
+            m = fmaxf(m, dpp_f<kDppXor2>(m)), s += dpp_f<kDppXor2>(s);
+            m = fmaxf(m, dpp_f<kDppHMirror>(m)), s += dpp_f<kDppHMirror>(s);
+            m = fmaxf(m, dpp_f<kDppMirror>(m)), s += dpp_f<kDppMirror>(s);
+            hsum[pg][r] = s;
+            if (i == 0) {
+              wred[wave][16 * pg + 4 * g + r] = m;
+              if (NT == 2) wsum[wave][16 * pg + 4 * g + r] = s;  // half a sub-block
+            }
+          }
+        __syncthreads();  // the magnitudes are in place and every wave is done with the stages
+        // element 16 el + i of the super-block, el = kTM wave + t: sub-block el / 2, i.e. h = el / 8,
+        // g = 2 (el / 4 % 2) + el % 2, hl = el / 2 % 2, u = i / 8
+        auto at = [&](int el) {
+          return (4 * (el >> 3) + 2 * (i >> 3) + ((el >> 1) & 1)) * 128 + ((el >> 1) & 2) * 16 + (el & 1) * 16 + kQPerm[i & 7] * 2;
+        };
+#pragma unroll
+        for (int pg = 0; pg < NPG; ++pg) {
+          f32x4 m4 = *reinterpret_cast<const f32x4*>(&wred[0][16 * pg + 4 * g]);
+#pragma unroll
+          for (int v = 1; v < NW; ++v) {
+            const f32x4 o4 = *reinterpret_cast<const f32x4*>(&wred[v][16 * pg + 4 * g]);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) m4[r] = fmaxf(m4[r], o4[r]);
+          }
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int pl = 16 * pg + 4 * g + r;
+            float p, pinv;
+            pow2_scale(m4[r], p, pinv);
+            uint8_t* im = &lds[pl * kEpRow];
+#pragma unroll
+            for (int t = 0; t < kTM; ++t) {
+              uint32_t h, l;
+              split2(hv[t][pg][r] * p, h, l);
+              uint8_t* d = im + at(kTM * wave + t);
+              *reinterpret_cast<uint16_t*>(d) = (uint16_t)h;
+              *reinterpret_cast<uint16_t*>(d + 64) = (uint16_t)l;
+            }
+            const int sub = kTM * wave / 2;  // its sums: NT = 2: with the next wave's half
+            if (i < 4 && (kTM == 2 || wave % 2 == 0)) {
+              const float X = NT == 2 ? hsum[pg][r] + wsum[(NW > 1 ? wave + 1 : 0) % NW][pl] : hsum[pg][r];
+              *reinterpret_cast<uint16_t*>(im + 1024 + i * 16 + kQPerm[sub] * 2) = (uint16_t)sum_term(X * p, i);
+            }
+            if (wave == 0 && i == 0 && pl < np) q.hpinv[(size_t)(p0 + pl) * (M >> 8) + rt] = pinv;
           }
         }
-      __syncthreads();  // the magnitudes are in place and every wave is done with the stages
-      // element 16 el + i of the super-block, el = kTM wave + t: sub-block el / 2, i.e. h = el / 8,
-      // g = 2 (el / 4 % 2) + el % 2, hl = el / 2 % 2, u = i / 8
-      auto at = [&](int el) {
-        return (4 * (el >> 3) + 2 * (i >> 3) + ((el >> 1) & 1)) * 128 + ((el >> 1) & 2) * 16 + (el & 1) * 16 + kQPerm[i & 7] * 2;
-      };
-#pragma unroll
-      for (int pg = 0; pg < NPG; ++pg) {
-        f32x4 m4 = *reinterpret_cast<const f32x4*>(&wred[0][16 * pg + 4 * g]);
-#pragma unroll
-        for (int v = 1; v < NW; ++v) {
-          const f32x4 o4 = *reinterpret_cast<const f32x4*>(&wred[v][16 * pg + 4 * g]);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) m4[r] = fmaxf(m4[r], o4[r]);
+        __syncthreads();
+        constexpr int kPieces = kQImgSb / 16;
+        for (int c = tid; c < np * kPieces; c += NW * 64) {
+          const int pl = c / kPieces, o = (c - pl * kPieces) * 16;
+          *reinterpret_cast<i32x4*>(q.himg + ((size_t)(p0 + pl) * (M >> 8) + rt) * kQImgSb + o) =
+              *reinterpret_cast<const i32x4*>(&lds[pl * kEpRow + o]);
         }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int pl = 16 * pg + 4 * g + r;
-          float p, pinv;
-          pow2_scale(m4[r], p, pinv);
-          uint8_t* im = &lds[pl * kEpRow];
-#pragma unroll
-          for (int t = 0; t < kTM; ++t) {
-            uint32_t h, l;
-            split2(hv[t][pg][r] * p, h, l);
-            uint8_t* d = im + at(kTM * wave + t);
-            *reinterpret_cast<uint16_t*>(d) = (uint16_t)h;
-            *reinterpret_cast<uint16_t*>(d + 64) = (uint16_t)l;
-          }
-          const int sub = kTM * wave / 2;  // its sums: NT = 2: with the next wave's half
-          if (i < 4 && (kTM == 2 || wave % 2 == 0)) {
-            const float X = NT == 2 ? hsum[pg][r] + wsum[(NW > 1 ? wave + 1 : 0) % NW][pl] : hsum[pg][r];
-            *reinterpret_cast<uint16_t*>(im + 1024 + i * 16 + kQPerm[sub] * 2) = (uint16_t)sum_term(X * p, i);
-          }
-          if (wave == 0 && i == 0 && pl < np) q.hpinv[(size_t)(p0 + pl) * (M >> 8) + rt] = pinv;
-        }
-      }
-      __syncthreads();
-      constexpr int kPieces = kQImgSb / 16;
-      for (int c = tid; c < np * kPieces; c += NW * 64) {
-        const int pl = c / kPieces, o = (c - pl * kPieces) * 16;
-        *reinterpret_cast<i32x4*>(q.himg + ((size_t)(p0 + pl) * (M >> 8) + rt) * kQImgSb + o) =
-            *reinterpret_cast<const i32x4*>(&lds[pl * kEpRow + o]);
       }
     }
   };
@@ -630,6 +670,43 @@ bool grouped_q4k_supported(const mr_layer& L) {
   return true;
 }
 
+// One grouped GEMM launch over at most `tiles` routed and `sh_tiles` shared pair tiles.
+template <bool GATEUP, int PG, int NW>
+static void launch_q4(const Launch& K, const GQ4Args& a, uint64_t tiles, uint64_t sh_tiles) {
+  constexpr int rows = q4_rows(GATEUP, PG, NW);
+  const dim3 grid(grouped_grid((uint64_t)(a.r.M / rows) * tiles + (uint64_t)(a.s.M / rows) * sh_tiles));
+  hipLaunchKernelGGL((k_grouped_q4k<GATEUP, PG, NW>), grid, dim3(64 * NW), 0, K.s, a);
+}
+
+// Pairs per tile and waves (of 16 rows) per gate/up item of a call.
+struct Q4Items {
+  int tile, gu_waves;
+};
+// With items(tile, rows) the expected number of gate/up work items (about half the experts hold a
+// part-filled tile more than their pairs fill). Measured (the whole call, us), 16-pair tiles / 64-pair
+// tiles unless said otherwise:
+// - 64 pairs read and unpack an expert's weights once for up to four 16-pair groups; they pay from a mean of
+//   16 to 30 pairs per expert on: 128 experts of 768 x 2048, top 8, mean 16 181 / 195, 24 212 / 218, 32
+//   253 / 234, 64 397 / 373; 512 experts of 512 x 2048, top 10, mean 20 534 / 538 and, with popularity
+//   ~ rank^-1.1, 418 / 384. So the line is 16, where a skewed batch gains what an even one loses.
+// - But an item of 64 pairs x 256 rows takes 35 us and more, and alone on its CU gains nothing: below half an
+//   item per CU the 16-pair tiles win at any mean (16 experts of 512 x 2048, top 4: 48 items 71 / 110, 80
+//   96 / 119, 112 119 / 123, 144 144 / 139, 208 197 / 157; 16 of 256 x 2048, top 2, 96 tokens: 44 / 69).
+// - 16-pair gate/up items of 8 waves or of 4 (128 or 64 rows): the latter while 128 rows would be less than an
+//   item per CU (102 items of 128 rows: 4 waves 48, 8 waves 51; 236: 72 / 78; 432: 92 / 88; 360: 83 / 81). Items of
+//   256 rows that split h themselves save k_split_h but leave CUs idle and are slower or equal everywhere:
+//   2 tokens of the first layer 62 us, with 64 rows 48; 8 tokens of 16 experts of 256 x 2048 51 / 39; 64 tokens
+//   of the first layer 146, with 128 rows 129; at best (32 tokens of 60 experts of 1024 x 2048 with a shared
+//   one) 77 / 77.
+static Q4Items q4_items(uint64_t T, uint64_t k, uint64_t E, uint64_t I, uint64_t Ish) {
+  const uint64_t P = T * k;
+  auto items = [&](uint64_t tile, uint64_t rows) {
+    return I / rows * (P / tile + std::min(P, E / 2)) + Ish / rows * ((T + tile - 1) / tile);
+  };
+  if (P > 16 * E && items(64, 256) >= 128) return {64, 16};
+  return {16, items(16, 128) >= 256 ? 8 : 4};
+}
+
 hipError_t launch_grouped_q4k(const Launch& K, const mr_layer& L, const float* x, uint32_t T, const int32_t* idx,
                               const float* w, float* y, void* scratch, const float* resid) {
   const int k = (int)L.d.top_k, E = (int)L.E, H = (int)L.H, I = (int)L.I, Ish = L.d.sh_gate ? (int)L.Ish : 0;
@@ -651,12 +728,8 @@ hipError_t launch_grouped_q4k(const Launch& K, const mr_layer& L, const float* x
   auto f32_at = [&](uint64_t o) { return reinterpret_cast<float*>(b + o); };
   auto i32_at = [&](uint64_t o) { return reinterpret_cast<int32_t*>(b + o); };
   auto u8_at = [&](uint64_t o) { return reinterpret_cast<uint8_t*>(b + o); };
-  // Pairs per tile: 16 while the experts' mean is at most 8, so that few experts need a second
-  // tile (which reads the expert's weights again), else 64: the 16-pair kernels keep twice the
-  // weight bytes in flight (128 pairs of 128 experts: gate/up 50 against 75 us, 3,840 of 512: 225
-  // against 303), and past 16 pairs every further tile costs them what the first did.
-  const bool small = (uint64_t)P <= 8ull * (uint64_t)E;
-  const int tile = small ? 16 : 64;
+  const Q4Items c = q4_items((uint64_t)T, (uint64_t)k, (uint64_t)E, (uint64_t)I, (uint64_t)Ish);
+  const int tile = c.tile;
   const GroupOut go{i32_at(p.pair_tok), f32_at(p.pair_w),   i32_at(p.pair_of), i32_at(p.exp_off),
                     i32_at(p.tile_off), i32_at(p.tile_exp), i32_at(p.hist)};
   hipError_t e;
@@ -683,11 +756,19 @@ hipError_t launch_grouped_q4k(const Launch& K, const mr_layer& L, const float* x
   a.E = E, a.alpha = L.d.alpha, a.limit = L.d.limit;
   {
     ProfScope ps(K, "grouped_q4k_gateup");
-    const dim3 grid(grouped_grid((uint64_t)(I / 256) * tiles + (uint64_t)(Ish / 256) * sh_tiles));
-    if (small)
-      hipLaunchKernelGGL((k_grouped_q4k<true, 1>), grid, dim3(64 * q4_waves(true, 1)), 0, K.s, a);
+    if (tile == 64)
+      launch_q4<true, 4, 16>(K, a, tiles, sh_tiles);
+    else if (c.gu_waves == 8)
+      launch_q4<true, 1, 8>(K, a, tiles, sh_tiles);
     else
-      hipLaunchKernelGGL((k_grouped_q4k<true, 4>), grid, dim3(64 * q4_waves(true, 4)), 0, K.s, a);
+      launch_q4<true, 1, 4>(K, a, tiles, sh_tiles);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
+  if (tile != 64) {
+    ProfScope ps(K, "split_h");
+    const int64_t n0 = (int64_t)P * (I / 256), n1 = (int64_t)T * (Ish / 256);
+    hipLaunchKernelGGL(k_split_h, dim3((unsigned)((n0 + n1 + 3) / 4)), dim3(256), 0, K.s, u8_at(p.himg), f32_at(p.hp), n0,
+                       Ish ? u8_at(p.hsimg) : nullptr, Ish ? f32_at(p.hsp) : nullptr, n1);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   GQ4Args d{};
@@ -701,11 +782,10 @@ hipError_t launch_grouped_q4k(const Launch& K, const mr_layer& L, const float* x
   d.exp_off = go.exp_off, d.tile_off = go.tile_off, d.tile_exp = go.tile_exp, d.E = E;
   {
     ProfScope ps(K, "grouped_q4k_down");
-    const dim3 grid(grouped_grid((uint64_t)((H + 255) / 256) * (tiles + sh_tiles)));
-    if (small)
-      hipLaunchKernelGGL((k_grouped_q4k<false, 1>), grid, dim3(64 * q4_waves(false, 1)), 0, K.s, d);
+    if (tile == 64)
+      launch_q4<false, 4, 4>(K, d, tiles, sh_tiles);
     else
-      hipLaunchKernelGGL((k_grouped_q4k<false, 4>), grid, dim3(64 * q4_waves(false, 4)), 0, K.s, d);
+      launch_q4<false, 1, 4>(K, d, tiles, sh_tiles);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   return launch_combine(K, f32_at(p.xo), go.pair_of, idx, w, L.d.down_bias, T, k, H, Ish ? f32_at(p.osh) : nullptr, sig,

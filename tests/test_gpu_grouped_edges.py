@@ -1,6 +1,6 @@
 """The grouped multi-token kernels at the edges of their tiles: pair counts around the 16-, 32- and
 64-pair tiles and their 16-pair groups (all tokens on the same experts, so an expert's pairs are
-the tokens), means that select either pair tile, one and several super-blocks per row, row counts
+the tokens), calls that select each pair tile and row count per work item, one and several super-blocks per row, row counts
 that fill half a tile, the shared expert's own width, and enough pairs for the grouping to take
 several workgroups. Reference: the per-token VALU path (f32 arithmetic, 3e-7 of the output), per
 token, max error over the token's largest output. Bar 2e-5 for Q4_K: the activations carry 22
@@ -32,18 +32,26 @@ def _batched(gpu_ctx, dl, x, kernel):
         dx.free(), dy.free()
 
 
+def _one_route(host, spec):
+    """The router bias decides: every token takes the same top_k experts."""
+    host["router_b"] = (host["router_b"] + 1e3 * (np.arange(spec.n_experts) % 5 == 1)
+                        - np.arange(spec.n_experts)).astype(np.float32)
+    return host
+
+
+def _check_layer(gpu_ctx, dl, T, bar=BAR):
+    x = W.x_tokens(dl.spec, T)
+    ref = _batched(gpu_ctx, dl, x, M.DECODE_VALU)
+    got = _batched(gpu_ctx, dl, x, M.DECODE_AUTO)
+    err = np.abs(got - ref).max(1) / np.abs(ref).max(1)
+    assert np.isfinite(got).all() and err.max() <= bar, (dl.spec, T, float(err.max()), int(err.argmax()))
+
+
 def _check(gpu_ctx, spec, T, one_route=False, bar=BAR):
     host = W.host_layer(spec)
-    if one_route:  # the bias decides: every token takes the same top_k experts
-        host["router_b"] = (host["router_b"] + 1e3 * (np.arange(spec.n_experts) % 5 == 1)
-                            - np.arange(spec.n_experts)).astype(np.float32)
-    dl = W.DeviceLayer(gpu_ctx, spec, host=host)
+    dl = W.DeviceLayer(gpu_ctx, spec, host=_one_route(host, spec) if one_route else host)
     try:
-        x = W.x_tokens(spec, T)
-        ref = _batched(gpu_ctx, dl, x, M.DECODE_VALU)
-        got = _batched(gpu_ctx, dl, x, M.DECODE_AUTO)
-        err = np.abs(got - ref).max(1) / np.abs(ref).max(1)
-        assert np.isfinite(got).all() and err.max() <= bar, (spec, T, float(err.max()), int(err.argmax()))
+        _check_layer(gpu_ctx, dl, T, bar)
     finally:
         dl.close()
 
@@ -53,9 +61,54 @@ def test_q4k_pairs_per_expert(gpu_ctx, T):
     _check(gpu_ctx, Q4, T, one_route=True)
 
 
-@pytest.mark.parametrize("T", [64, 65])  # mean pairs per expert 8 and just above: the pair tile changes
+@pytest.mark.parametrize("T", [64, 65])  # 8 pairs per expert in the mean and just above
 def test_q4k_pair_tile_rule(gpu_ctx, T):
     _check(gpu_ctx, Q4, T)
+
+
+# 10 super-blocks of 256 gate rows, 3 super-blocks per gate/up row and 10 per down row; every token on the same
+# three of 12 experts. Gate/up items of 64 rows up to 37 tokens, of 128 rows up to 149 (16-pair tiles both),
+# then 64-pair tiles of 256 rows, whose last tile holds 1, 2, 3 or 4 16-pair groups.
+WIDE = replace(Q4, hidden=768, inter=2560, n_experts=12)
+
+
+@pytest.fixture(scope="module", params=[0, 256], ids=["routed", "shared"])
+def wide_layer(gpu_ctx, request):
+    spec = replace(WIDE, sh_inter=request.param)
+    dl = W.DeviceLayer(gpu_ctx, spec, host=_one_route(W.host_layer(spec), spec))
+    yield dl
+    dl.close()
+
+
+@pytest.mark.parametrize("T", [1, 15, 16, 17, 33, 37, 38, 47, 48, 49, 64, 65, 149, 160, 161, 176, 177, 191, 192, 193,
+                               207, 208, 209])
+def test_q4k_work_items(gpu_ctx, wide_layer, T):
+    _check_layer(gpu_ctx, wide_layer, T)
+
+
+def _ran(gpu_ctx, dl, T, scope):
+    """Launches named `scope` in a batched call of T tokens."""
+    gpu_ctx.profile_reset()
+    gpu_ctx.set_option(M.OPT_PROFILE, 1)
+    try:
+        _batched(gpu_ctx, dl, W.x_tokens(dl.spec, T), M.DECODE_AUTO)
+        return gpu_ctx.profile_read(scope)[0]
+    finally:
+        gpu_ctx.set_option(M.OPT_PROFILE, 0)
+
+
+# Few tokens, and many tokens of few narrow experts: 24 and 16 items of 256 rows, or 24 of 64 pairs and 256
+# rows, leave nine in ten CUs idle (28, 31 and 81% slower than smaller items). Smaller items pass h through
+# memory (split_h); with an item for every second CU they need not be smaller.
+@pytest.mark.parametrize("E,k,H,I,T,small", [(128, 8, 2048, 768, 1, True), (16, 2, 2048, 256, 8, True),
+                                             (16, 2, 2048, 256, 512, True), (12, 3, 768, 2560, 160, False)])
+def test_q4k_few_work_items_are_split(gpu_ctx, E, k, H, I, T, small):
+    spec = replace(Q4, hidden=H, inter=I, n_experts=E, top_k=k)
+    dl = W.DeviceLayer(gpu_ctx, spec)
+    try:
+        assert _ran(gpu_ctx, dl, T, "split_h") == (1 if small else 0)
+    finally:
+        dl.close()
 
 
 @pytest.mark.parametrize("H,I,sh", [(256, 256, 0), (768, 512, 256), (1280, 768, 1024), (2048, 256, 512)])
