@@ -192,9 +192,11 @@ struct GQ4Args {
 // Work item: (expert e, rows of each matrix, tile of 16 PG pairs), NW waves. Gate/up: wave w rows
 // 16 w .. 16 w + 15 of the gate and of the up matrix, so that a lane holds both values of a
 // (row, pair). NW = 16, 256 rows: a down input super-block forms inside one item, which splits it;
-// NW = 8 or 4: h goes through memory, for k_split_h. Down: 4 waves of 32 rows (PG = 1) or of 64 (PG = 4:
-// 323 us at the size below, with 8 of 32 rows 348, as its accumulators fit there). Which of them runs:
-// see launch_grouped_q4k. The activations are the MFMA's A operand (rows:
+// NW = 8 or 4: h goes through memory, for k_split_h. (Two tiles of each matrix in eight waves, so that a
+// fragment read serves four MFMAs, PG = 4: the whole call 941 -> 926 us at the size below, but 161 -> 171 us
+// for 1,024 tokens of 16 experts of 1024 x 3072, and 3% slower at 512 to 1,024 tokens of the size below.)
+// Down: 4 waves of 32 rows (PG = 1) or of 64 (PG = 4: 323 us at the size below, with 8 of 32 rows 348, as
+// its accumulators fit there). Which of them runs: see q4_items. The activations are the MFMA's A operand (rows:
 // pairs), the weights its B operand (columns: weight rows): lane (i, g) = lane % 16, lane / 16
 // holds weight row i of every tile, and of D weight row i for pairs 4g .. 4g+3 of each pair group.
 //   A wave's weights come in halves of a super-block, 64 bytes per row, one or two halves ahead in
@@ -218,11 +220,12 @@ constexpr int q4_tiles(bool gateup, int pg) { return gateup || pg == 1 ? 2 : 4; 
 constexpr int q4_rows(bool gateup, int pg, int waves) { return 16 * q4_tiles(gateup, pg) / (gateup ? 2 : 1) * waves; }
 
 template <bool GATEUP, int PG, int NW>
-__global__ __launch_bounds__(64 * NW, q4_tiles(GATEUP, PG) == 4 ? 2 : 4) void k_grouped_q4k(GQ4Args a) {
+__global__ __launch_bounds__(64 * NW, q4_tiles(GATEUP, PG) == 4 ? 2 : NW == 4 ? 3 : 4) void k_grouped_q4k(GQ4Args a) {
   constexpr int NT = q4_tiles(GATEUP, PG), kRows = q4_rows(GATEUP, PG, NW);
   static_assert(256 % kRows == 0, "row counts are multiples of 256");
   constexpr bool kSplit = GATEUP && kRows == 256;  // the epilogue writes images
   constexpr int kTM = GATEUP ? NT / 2 : NT;  // tiles of one matrix per wave
+  static_assert(!kSplit || kTM == 1, "the split takes 16 rows of a matrix per wave: half a sub-block");
   constexpr int kPF = PG == 1 ? 2 : 1;       // half super-blocks of weights in flight
   constexpr int kKS = PG == 1 ? 8 : 2;       // K steps per stage
   constexpr int kNS = 8 / kKS;               // stages per super-block
@@ -237,7 +240,7 @@ __global__ __launch_bounds__(64 * NW, q4_tiles(GATEUP, PG) == 4 ? 2 : 4) void k_
   __shared__ __align__(16) uint8_t hst[NW][NT * 256];   // and their headers: [tile][row][16 bytes]
   __shared__ __align__(16) float pst[2][kPairs];       // down: 1/p of (pair, super-block); gate/up: [0] of the pair
   __shared__ __align__(16) float pw[kPairs];           // GATEUP: routing weights
-  __shared__ __align__(16) float wred[kSplit ? NW : 1][kPairs], wsum[kSplit && NT == 2 ? NW : 1][kPairs];
+  __shared__ __align__(16) float wred[kSplit ? NW : 1][kPairs], wsum[kSplit ? NW : 1][kPairs];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -493,7 +496,6 @@ __global__ __launch_bounds__(64 * NW, q4_tiles(GATEUP, PG) == 4 ? 2 : 4) void k_
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         const int row = wrow0 + 16 * t + i;
-        if (row >= M) continue;
 #pragma unroll
         for (int pg = 0; pg < NPG; ++pg)
 #pragma unroll
@@ -544,7 +546,7 @@ __global__ __launch_bounds__(64 * NW, q4_tiles(GATEUP, PG) == 4 ? 2 : 4) void k_
         for (int pg = 0; pg < NPG; ++pg)
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            float m = fmaxf(fabsf(hv[0][pg][r]), fabsf(hv[kTM - 1][pg][r])), s = kTM == 2 ? hv[0][pg][r] + hv[kTM - 1][pg][r] : hv[0][pg][r];
+            float m = fabsf(hv[0][pg][r]), s = hv[0][pg][r];
             m = fmaxf(m, dpp_f<kDppXor1>(m)), s += dpp_f<kDppXor1>(s);
             m = fmaxf(m, dpp_f<kDppXor2>(m)), s += dpp_f<kDppXor2>(s);
             m = fmaxf(m, dpp_f<kDppHMirror>(m)), s += dpp_f<kDppHMirror>(s);
@@ -552,11 +554,11 @@ __global__ __launch_bounds__(64 * NW, q4_tiles(GATEUP, PG) == 4 ? 2 : 4) void k_
             hsum[pg][r] = s;
             if (i == 0) {
               wred[wave][16 * pg + 4 * g + r] = m;
-              if (NT == 2) wsum[wave][16 * pg + 4 * g + r] = s;  // half a sub-block
+              wsum[wave][16 * pg + 4 * g + r] = s;  // half a sub-block
             }
           }
         __syncthreads();  // the magnitudes are in place and every wave is done with the stages
-        // element 16 el + i of the super-block, el = kTM wave + t: sub-block el / 2, i.e. h = el / 8,
+        // element 16 el + i of the super-block, el = wave: sub-block el / 2, i.e. h = el / 8,
         // g = 2 (el / 4 % 2) + el % 2, hl = el / 2 % 2, u = i / 8
         auto at = [&](int el) {
           return (4 * (el >> 3) + 2 * (i >> 3) + ((el >> 1) & 1)) * 128 + ((el >> 1) & 2) * 16 + (el & 1) * 16 + kQPerm[i & 7] * 2;
@@ -576,17 +578,14 @@ __global__ __launch_bounds__(64 * NW, q4_tiles(GATEUP, PG) == 4 ? 2 : 4) void k_
             float p, pinv;
             pow2_scale(m4[r], p, pinv);
             uint8_t* im = &lds[pl * kEpRow];
-#pragma unroll
-            for (int t = 0; t < kTM; ++t) {
-              uint32_t h, l;
-              split2(hv[t][pg][r] * p, h, l);
-              uint8_t* d = im + at(kTM * wave + t);
-              *reinterpret_cast<uint16_t*>(d) = (uint16_t)h;
-              *reinterpret_cast<uint16_t*>(d + 64) = (uint16_t)l;
-            }
-            const int sub = kTM * wave / 2;  // its sums: NT = 2: with the next wave's half
-            if (i < 4 && (kTM == 2 || wave % 2 == 0)) {
-              const float X = NT == 2 ? hsum[pg][r] + wsum[(NW > 1 ? wave + 1 : 0) % NW][pl] : hsum[pg][r];
+            uint32_t h, l;
+            split2(hv[0][pg][r] * p, h, l);
+            uint8_t* d = im + at(wave);
+            *reinterpret_cast<uint16_t*>(d) = (uint16_t)h;
+            *reinterpret_cast<uint16_t*>(d + 64) = (uint16_t)l;
+            const int sub = wave / 2;
+            if (i < 4 && wave % 2 == 0) {  // its sums, with the next wave's half
+              const float X = hsum[pg][r] + wsum[(wave + 1) % NW][pl];
               *reinterpret_cast<uint16_t*>(im + 1024 + i * 16 + kQPerm[sub] * 2) = (uint16_t)sum_term(X * p, i);
             }
             if (wave == 0 && i == 0 && pl < np) q.hpinv[(size_t)(p0 + pl) * (M >> 8) + rt] = pinv;
