@@ -198,3 +198,39 @@ def test_q4k_scales_zero_and_denormal_rows(gpu_ctx):
             assert np.abs(got[t] - ref[t]).max() <= BAR * np.abs(ref[t]).max() + 1e-37, t
     finally:
         dl.close()
+
+
+def test_q4k_call_in_parts(gpu_ctx):
+    """More tokens than the images' 31-bit offsets cover (30,599 of hidden size 16,384) run in parts: every
+    token's result is that of the same row in a small call, without and with the residual, in place."""
+    H, n = 16384, 601
+    T = 0x7F000000 // (H // 256 * 1088) + 37
+    spec = replace(Q4, hidden=H, n_experts=7, top_k=2, sh_inter=256)
+    ctx = M.Context(0)  # its scratch goes with it
+    dl = W.DeviceLayer(ctx, spec, host=_one_route(W.host_layer(spec), spec))
+    try:
+        base = W.x_tokens(spec, n)
+        norm_w = ctx.to_device(W.norm_weights(1, H)[0])
+        dx = ctx.to_device(base)
+        want = ctx.alloc(n * H * 4)
+        dl.layer.forward_batched(dx, n, want)
+        dl.layer.forward_batched_residual(dx, n, norm_w, 1e-5, dx)
+        ctx.sync()
+        plain, resid = (b.download(np.float32).reshape(n, H) for b in (want, dx))
+        dx.free(), want.free()
+        rows = np.arange(T) % n
+        dx, dy = ctx.to_device(base[rows]), ctx.alloc(T * H * 4)
+        dl.layer.forward_batched(dx, T, dy)
+        dl.layer.forward_batched_residual(dx, T, norm_w, 1e-5, dx)
+        ctx.sync()
+        for buf, ref in ((dy, plain), (dx, resid)):
+            got = buf.download(np.float32).reshape(T, H)
+            for t0 in range(0, T, n):  # block by block: the whole is 2 GB
+                g = got[t0:t0 + n]
+                r = ref[:g.shape[0]]
+                assert (np.abs(g - r).max(1) <= BAR * np.abs(r).max(1)).all(), t0
+        for b in (dx, dy, norm_w):
+            b.free()
+    finally:
+        dl.close()
+        ctx.close()
