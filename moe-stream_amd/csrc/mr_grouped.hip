@@ -25,6 +25,7 @@
 #include "mr_mx_mfma.h"
 
 #include <algorithm>
+#include <cmath>
 #include <climits>
 #include <type_traits>
 
@@ -744,26 +745,50 @@ static hipError_t launch_gemm(const Launch& K, const GroupedArgs& a, int pg, uin
   return hipGetLastError();
 }
 
-// 16-pair groups per work item, for `pairs` pairs over `experts` experts with `rows` gate rows.
-// More groups reuse a step's weight windows and their alignment for more MFMAs; fewer waste less
-// on part-filled tiles and leave room for three workgroups per CU. The lines lie at a mean of 8
-// and 64 pairs per expert (whole call, us, 32 experts of 2880 x 2880, 1 / 2 / 4 groups: mean 4
-// 156 / 172 / 185; 8 162 / 176 / 195; 16 203 / 192 / 205; 64 370 / 308 / 298 and, with popularity
-// ~ rank^-1.1, 401 / 324 / 323 with a slower down launch; 128 620 / 492 / 447; 255 1166 / 911 / 780). Few work items take fewer groups, so that the CUs are not left idle: below two items per
-// CU 4 groups lose to 2 (16 experts of 1600 x 1504, 500 tokens of 4, 372 items: 113 / 109 us),
-// below one 2 lose to 1 (8 experts of 1024 x 512, 40 tokens of 4: 69 / 59 us).
-static int pair_groups(uint64_t pairs, uint64_t experts, int rows) {
-  int pg = pairs > 64 * experts ? 4 : pairs > 8 * experts ? 2 : 1;
+// 16-pair groups per work item, for `pairs` pairs over `experts` experts of `rows` gate rows and `hidden`
+// down rows. More groups reuse a step's weight windows and their alignment for more MFMAs; fewer waste less
+// on part-filled tiles and leave room for three workgroups per CU. The lines lie at a mean of 12 and 64
+// pairs per expert. Whole call, us, 32 experts of 2880 x 2880, 1 / 2 / 4 groups, even routing and
+// popularity ~ rank^-1.1:
+//   mean     even                  skewed
+//   8        162 / 176 / 192       151 / 169 / 176
+//   12       183 / 184 / 200
+//   16       204 / 194 / 206       218 / 195 / 225
+//   32       261 / 248 / 227       283 / 247 / 249
+//   64       374 / 309 / 300       408 / 332 / 333
+//   128      626 / 500 / 452       669 / 530 / 480
+//   255     1173 / 913 / 778
+// From 32 to 64 an even batch gains up to 8% by 4 groups, but a skewed one nothing, and its down launch
+// (fewer, longer items) loses: 110 -> 122 us at 64. Few work items take fewer groups, so that the CUs are
+// not left idle: below two items per CU 4 groups lose to 2 (16 experts of 1600 x 1504, 500 tokens of 4,
+// 372 items: 113 / 109 us), below seven for eight CUs 2 lose to 1 (24 experts of 1024 x 2048, 256 tokens of 3,
+// 192 items: 121 / 100 us; but 28 of 1152 x 2304, 128 tokens of 3, 252 items: 68 / 74).
+// Past that the rounds decide between 4 and 2 (512 workgroups are on the CUs at once; a part-filled
+// last round half counts, as rounds overlap). An item of 4 groups takes about 1.6 times as long as one of
+// 2; 1.4 leaves the choice at 4 where the estimate of the tiles is too coarse. 2 / 4 groups: 8 experts of
+// 2944 x 1152, 384 tokens of 4 111 / 129 us; 18 of 1920 x 1440, 1,200 tokens of 2 134 / 158; 12 of 2720 x
+// 1216, 2,048 tokens of 2 238 / 229 (but 1,536 tokens, a few items past two rounds, 182 / 203).
+static int pair_groups(uint64_t pairs, uint64_t experts, int rows, int hidden) {
+  int pg = pairs > 64 * experts ? 4 : pairs > 12 * experts ? 2 : 1;
   const uint64_t n_rt = (uint64_t)((rows + kRowsOf<true> - 1) / kRowsOf<true>);
-  while (pg > 1 && std::max(pairs / (16 * pg), std::min(pairs, experts)) * n_rt < 128u * pg) pg >>= 1;
-  return pg;
+  while (pg > 1 && std::max(pairs / (16 * pg), std::min(pairs, experts)) * n_rt < (pg == 4 ? 512u : 224u)) pg >>= 1;
+  if (pg < 4) return pg;
+  auto cost = [&](int g) {  // about half the experts hold a part-filled tile more than their pairs fill
+    const double tiles = (double)pairs / (16 * g) + 0.5 * (double)std::min(pairs, experts);
+    auto rounds = [&](uint64_t n) {
+      const double r = tiles * (double)n / 512;
+      return 0.5 * (std::max(r, 1.0) + std::ceil(r));
+    };
+    return rounds(n_rt) * hidden + rounds((uint64_t)((hidden + kRowsOf<false> - 1) / kRowsOf<false>)) * rows;
+  };
+  return 1.4 * cost(4) < cost(2) ? 4 : 2;
 }
 
 hipError_t launch_grouped(const Launch& K, const mr_layer& L, const float* x, uint32_t T, const int32_t* idx,
                           const float* w, float* y, const GroupedScratch& gs, const float* resid) {
   const int k = (int)L.d.top_k, E = (int)L.E, H = (int)L.H, I = (int)L.I;
   const int P = (int)T * k;
-  const int pg = pair_groups((uint64_t)P, (uint64_t)E, I), tile = 16 * pg;
+  const int pg = pair_groups((uint64_t)P, (uint64_t)E, I, H), tile = 16 * pg;
   const uint64_t max_tiles = group_tiles_max((uint64_t)P, (uint64_t)E, (uint64_t)tile);
   hipError_t e;
   const GroupOut go{gs.pair_tok, gs.pair_w, gs.pair_of, gs.exp_off, gs.tile_off, gs.tile_exp, gs.hist};
@@ -789,7 +814,7 @@ hipError_t launch_grouped(const Launch& K, const mr_layer& L, const float* x, ui
   // weight 1 and SiLU (the routed experts' activation does not apply), its down outputs
   // [T][H], then sigmoid(x . gate_inp) per token, which the combine applies after the routed
   // sum.
-  const int Ish = L.d.sh_gate ? (int)L.Ish : 0, pgs = pair_groups(T, 1, Ish), tiles = ((int)T + 16 * pgs - 1) / (16 * pgs);
+  const int Ish = L.d.sh_gate ? (int)L.Ish : 0, pgs = pair_groups(T, 1, Ish, H), tiles = ((int)T + 16 * pgs - 1) / (16 * pgs);
   if (Ish) {
     GroupedArgs sg{};
     sg.w0 = expert_loc(L.d.sh_gate), sg.w1 = expert_loc(L.d.sh_up);

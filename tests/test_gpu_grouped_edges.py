@@ -124,13 +124,19 @@ MX_BAR = 2.0 ** -11
 
 
 # 17 row tiles of the 2,080 gate rows (the last of 32 rows), 9 blocks per row of 288; every token on the
-# same three experts. 16-pair tiles up to 64 tokens (a mean of 8 pairs per expert), then 32-pair tiles,
-# 64-pair tiles from about 680 tokens on (512 work items); the counts leave the last tile around each
-# edge of its 16-pair groups.
+# same three experts. 16-pair tiles up to 96 tokens (a mean of 12 pairs per expert), then 32-pair tiles; the
+# counts leave the last tile around each edge of its 16-pair groups.
 @pytest.mark.parametrize("T", [1, 2, 15, 16, 17, 33, 64, 65, 80, 81, 96, 97, 256, 683, 704, 705, 720, 721, 735, 737,
                                753])
 def test_mxfp4_pairs_per_expert(gpu_ctx, T):
     _check(gpu_ctx, MX, T, one_route=True, bar=MX_BAR)
+
+
+# Two of six experts, 33 blocks per row: from about 1,900 tokens on 64-pair tiles, two rounds of work items.
+# The last tile around each edge of its 16-pair groups.
+@pytest.mark.parametrize("T", [1985, 2000, 2001, 2016, 2017, 2032, 2033, 2047, 2048])
+def test_mxfp4_64_pair_tiles(gpu_ctx, T):
+    _check(gpu_ctx, replace(MX, hidden=1056, n_experts=6, top_k=2), T, one_route=True, bar=MX_BAR)
 
 
 @pytest.mark.parametrize("H,I,sh", [(32, 32, 0), (160, 96, 0), (1056, 288, 2080), (2880, 160, 64)])
