@@ -479,23 +479,32 @@ __global__ __launch_bounds__(256) void k_gateup_valu(GateUpArgs a) {
   const uint64_t rb = row_bytes_of(TYPE, (uint64_t)a.H);
   const int row0 = blockIdx.x * 16 + wave * 4;
   if (row0 >= a.I) return;
-  const uint8_t* rows[8];  // 4 gate rows and the same up rows; past I the last row again, not stored
+  // R gate rows and the same up rows at a time. Q4_K with 4: 177 VGPRs, two waves per SIMD, which costs more
+  // than the shared reads give once there are many workgroups (experts of 256 tokens, us, R = 4 / 2 / rows one
+  // by one: 128 of 768 x 2048, 8 per token, 3064 / 2514 / 3207; 24 of 256 x 512, 3 per token, 272 / 235 / 234; 1 token
+  // of the former 38 / 38 / 57). MXFP4 with 4: 122 VGPRs.
+  constexpr int R = TYPE == MR_GGML_Q4_K ? 2 : 4;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const uint64_t off = (uint64_t)min(row0 + i, a.I - 1) * rb;
-    rows[i] = G + off, rows[4 + i] = U + off;
-  }
-  float d[8];
-  rows_dot<TYPE, 8>(rows, xs, a.xst, a.H, lane, d);
+  for (int i0 = 0; i0 < 4; i0 += R) {
+    if (i0) __builtin_amdgcn_sched_barrier(0);  // one after the other
+    const uint8_t* rows[2 * R];  // past I the last row again, not stored
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = row0 + i;
-    if (lane == 0 && r < a.I) {
-      float g = d[i], u = d[4 + i];
-      if (a.gate_b) g = g + a.gate_b[(size_t)e * a.I + r];
-      if (a.up_b) u = u + a.up_b[(size_t)e * a.I + r];
-      float h = a.act_kind == MR_ACT_SWIGLU_OAI ? swiglu_oai(g, u, a.alpha, a.limit) : silu_mul(g, u);
-      a.act[((size_t)t * a.k + slot) * a.I + r] = h;
+    for (int i = 0; i < R; ++i) {
+      const uint64_t off = (uint64_t)min(row0 + i0 + i, a.I - 1) * rb;
+      rows[i] = G + off, rows[R + i] = U + off;
+    }
+    float d[2 * R];
+    rows_dot<TYPE, 2 * R>(rows, xs, a.xst, a.H, lane, d);
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const int r = row0 + i0 + i;
+      if (lane == 0 && r < a.I) {
+        float g = d[i], u = d[R + i];
+        if (a.gate_b) g = g + a.gate_b[(size_t)e * a.I + r];
+        if (a.up_b) u = u + a.up_b[(size_t)e * a.I + r];
+        float h = a.act_kind == MR_ACT_SWIGLU_OAI ? swiglu_oai(g, u, a.alpha, a.limit) : silu_mul(g, u);
+        a.act[((size_t)t * a.k + slot) * a.I + r] = h;
+      }
     }
   }
 }
