@@ -1,10 +1,12 @@
-"""Multi-token Q4_K layers on the grouped int8-MFMA path (mr_moe_forward_batched and
+"""Multi-token Q4_K layers on the grouped f16-MFMA path (mr_moe_forward_batched and
 mr_moe_forward_batched_residual): every token against an oracle that follows the reference's
 multi-token CPU path (layer.rs:1449-1514: each expert's matrices dequantized once by the oracle's
 dequant_q4k, dequant.rs:218-262, then applied to all of the expert's tokens, here in float64; the
 shared expert and its sigmoid gate after the routed sum, layer.rs:1898-1953), and against the
-per-token VALU path. Bar: max relative error 1e-3 per token (2e-3 between the two GPU paths);
-tokens whose k-th and (k+1)-th router logits lie within 1e-5 of the largest are tie-ambiguous
+per-token VALU path. Bar: max relative error 2e-5 per token, also between the two GPU paths: the
+activations and h carry 22 significant bits (2^-22 each), the sums of up to 2,048 products are f32 (some
+2^-24 of the products' magnitudes each, 3e-7 together), the routing weights agree to some 1e-6 (4.2e-6 at
+most here). Without the second f16 term the error is 2^-12 per element, ten times the bar. Tokens whose k-th and (k+1)-th router logits lie within 1e-5 of the largest are tie-ambiguous
 and skipped. Routing (indices exactly, weights to 1e-5) is compared with the oracle's
 top_k_routing on the oracle's logits.
 """
@@ -20,7 +22,8 @@ from moe_rocm import workloads as W
 
 pytestmark = pytest.mark.gpu
 
-REL_TOL = 1e-3
+REL_TOL = 2e-5
+MX_TOL = 1e-3  # MXFP4: three e4m3 terms, 2^-12 of a block's largest value in each product
 
 TINY_SH = W.LayerSpec(260, 0, W.GGML_Q4_K, 512, 256, 24, 5, W.ROUTE_NORM_TOPK, W.ACT_SILU, False, False,
                       sh_inter=256)
@@ -163,7 +166,7 @@ def _check(gpu_ctx, dl, host, x, valu=True, min_checked=0.9):
         assert np.allclose(np.sort(gw[t]), np.sort(rw[t]), rtol=1e-5, atol=1e-6), t
         assert rel_err(y[t], ry[t]) <= REL_TOL, (t, rel_err(y[t], ry[t]))
         if valu:
-            assert rel_err(y[t], yv[t]) <= 2 * REL_TOL, (t, rel_err(y[t], yv[t]))
+            assert rel_err(y[t], yv[t]) <= REL_TOL, (t, rel_err(y[t], yv[t]))
         checked += 1
     assert checked >= min_checked * T
     return y
@@ -235,7 +238,7 @@ def test_batched_residual_mxfp4(gpu_ctx, built):
         if _ambiguous(lg[0], spec.top_k):
             continue
         err = np.abs(got[t].astype(np.float64) - ref[0]).max() / np.abs(ref[0].astype(np.float64) - h[t]).max()
-        assert err <= REL_TOL, (t, err)
+        assert err <= MX_TOL, (t, err)
 
 
 def test_grouped_q4k_noalloc_and_graph_match_batched(gpu_ctx, built):
