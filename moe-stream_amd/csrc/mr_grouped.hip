@@ -554,9 +554,10 @@ __global__ __launch_bounds__(256, kPG == 1 ? 3 : 2) void k_grouped_gemm(GroupedA
 // o[pair][row] + w * b_down[e][row], then + sig[t] * o_sh[t][row] when a shared expert ran
 // (layer.rs:1935-1951); with a residual input, y = resid + that (layer.rs:462-473; resid may be y:
 // a thread reads what it overwrites). Added here it costs one read of h; as a launch of its own it
-// read the sum back and wrote it again (2,039 tokens of 2880: 16 us after this kernel's 20; 4: 4.7). One thread per (token, 4 rows) on a (row groups, tokens) grid (tokens
-// past gridDim.y loop); the token's (at most KM) pair indices stay in registers and are taken
-// smallest first, and all of a thread's loads issue before the sums. H % 4 == 0.
+// read the sum back and wrote it again (2,039 tokens of 2880: 16 us after this kernel's 20; 4: 4.7).
+// One thread per (token, 4 rows) on a (row groups, tokens) grid (tokens past gridDim.y loop); the
+// token's (at most KM) pair indices stay in registers and are taken smallest first, and all of a
+// thread's loads issue before the sums. H % 4 == 0.
 template <int KM>
 __global__ __launch_bounds__(256) void k_combine(const float* __restrict__ o, const int32_t* __restrict__ pair_of,
                                                  const int32_t* __restrict__ idx, const float* __restrict__ w,

@@ -356,9 +356,12 @@ hipError_t launch_topk(const Launch& K, const float* logits, uint32_t T, uint32_
 // xst floats apart. Each lane adds up its units (every 64th block of 32 elements) in order; the
 // lanes' partial sums are acc. Units and the order of every sum are the same for any R, so a row's
 // result does not depend on the rows beside it.
-// The vector bounds it: a unit reads 128 bytes of it for 17 or 18 bytes of weights, so R rows share
-// a read, and with xst = 36 the lanes' blocks start in different banks (at 32 all in one: experts of
-// 8 tokens, 32 of 2880 x 2880, gate/up 148 us and down 105 us; now 104 and 68 us).
+// A unit reads 128 bytes of the vector for 17 or 18 bytes of weights, so R rows share a read, and with
+// xst = 36 the lanes' blocks start in different banks (at 32 all in one): one row at a time the vector's reads
+// bounded it (experts of 8 tokens, 32 of 2880 x 2880, gate/up 148 us and down 105 us; now 104 and 68 us).
+// What bounds it now: the latency of the weight loads, one 17-byte window per lane and row, 90 units on 64
+// lanes in two rounds. Of the waves' time 67% (gate/up) and 72% (down) is waiting, 0.1% of it for LDS; VALU
+// issue takes 17 and 12% of the SIMDs' cycles.
 constexpr int kXStride = 36;
 
 // MXFP4: unit = one 17-byte block; sum_b d_b * sum_j kvalue_j x_j.
