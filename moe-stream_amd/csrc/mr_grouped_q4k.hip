@@ -541,7 +541,6 @@ __global__ __launch_bounds__(64 * NW, q4_tiles(GATEUP, PG) == 4 ? 2 : NW == 4 ? 
         // The item's 256 rows of a pair, one super-block, are split. Largest magnitudes and sums go
         // over the 16 lanes of a row group, the magnitudes over the waves through LDS; the halves
         // are put in place in LDS and leave as whole 16-byte pieces.
-        float hsum[NPG][4];
 #pragma unroll
         for (int pg = 0; pg < NPG; ++pg)
 #pragma unroll
@@ -551,7 +550,6 @@ __global__ __launch_bounds__(64 * NW, q4_tiles(GATEUP, PG) == 4 ? 2 : NW == 4 ? 
             m = fmaxf(m, dpp_f<kDppXor2>(m)), s += dpp_f<kDppXor2>(s);
             m = fmaxf(m, dpp_f<kDppHMirror>(m)), s += dpp_f<kDppHMirror>(s);
             m = fmaxf(m, dpp_f<kDppMirror>(m)), s += dpp_f<kDppMirror>(s);
-            hsum[pg][r] = s;
             if (i == 0) {
               wred[wave][16 * pg + 4 * g + r] = m;
               wsum[wave][16 * pg + 4 * g + r] = s;  // half a sub-block
@@ -584,8 +582,12 @@ __global__ __launch_bounds__(64 * NW, q4_tiles(GATEUP, PG) == 4 ? 2 : NW == 4 ? 
             *reinterpret_cast<uint16_t*>(d) = (uint16_t)h;
             *reinterpret_cast<uint16_t*>(d + 64) = (uint16_t)l;
             const int sub = wave / 2;
-            if (i < 4 && wave % 2 == 0) {  // its sums, with the next wave's half
-              const float X = hsum[pg][r] + wsum[(wave + 1) % NW][pl];
+            // its sum, of this wave's half and the next one's. Four lanes write the terms of one value: both
+            // halves come from LDS, since the lanes' own sums may differ in the last bit (the compiler fuses
+            // the routing weight's product into the first addition), and a sum whose f16 rounding parts two
+            // lanes would be off by 2^-11.
+            if (i < 4 && wave % 2 == 0) {
+              const float X = wsum[wave][pl] + wsum[(wave + 1) % NW][pl];
               *reinterpret_cast<uint16_t*>(im + 1024 + i * 16 + kQPerm[sub] * 2) = (uint16_t)sum_term(X * p, i);
             }
             if (wave == 0 && i == 0 && pl < np) q.hpinv[(size_t)(p0 + pl) * (M >> 8) + rt] = pinv;

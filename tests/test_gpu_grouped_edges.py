@@ -86,6 +86,26 @@ def test_q4k_work_items(gpu_ctx, wide_layer, T):
     _check_layer(gpu_ctx, wide_layer, T)
 
 
+def test_q4k_sub_block_sums(gpu_ctx):
+    """A down matrix of minimums alone: row 8 b + j is minus the sum of h over sub-block j of super-block b.
+    Each sum goes to the down kernel as three f16 terms, which several lanes write: some 300,000 sums, so that
+    many lie where two lanes' roundings of the same sum could part (2^-11 of it then, fifty times the bar)."""
+    H, nsb, E = WIDE.hidden, WIDE.inter // 256, WIDE.n_experts
+    host = W.host_layer(WIDE)
+    down = np.zeros((E, H, nsb, 144), np.uint8)
+    for b in range(nsb):
+        for j in range(8):
+            down[:, 8 * b + j, b, 2:4] = np.frombuffer(np.float16(1).tobytes(), np.uint8)  # dmin
+            down[:, 8 * b + j, b, 8 + j] = 1 if j < 4 else 16  # m_j = 1
+    host["down"] = down.reshape(-1)
+    dl = W.DeviceLayer(gpu_ctx, WIDE, host=host)
+    try:
+        for T in (30, 60, 1400):  # each kind of work item
+            _check_layer(gpu_ctx, dl, T)
+    finally:
+        dl.close()
+
+
 def _ran(gpu_ctx, dl, T, scope):
     """Launches named `scope` in a batched call of T tokens."""
     gpu_ctx.profile_reset()

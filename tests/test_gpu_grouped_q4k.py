@@ -5,8 +5,9 @@ dequant_q4k, dequant.rs:218-262, then applied to all of the expert's tokens, her
 shared expert and its sigmoid gate after the routed sum, layer.rs:1898-1953), and against the
 per-token VALU path. Bar: max relative error 2e-5 per token, also between the two GPU paths: the
 activations and h carry 22 significant bits (2^-22 each), the sums of up to 2,048 products are f32 (some
-2^-24 of the products' magnitudes each, 3e-7 together), the routing weights agree to some 1e-6 (4.2e-6 at
-most here). Without the second f16 term the error is 2^-12 per element, ten times the bar. Tokens whose k-th and (k+1)-th router logits lie within 1e-5 of the largest are tie-ambiguous
+2^-24 of the products' magnitudes each, 3e-7 together), the routing weights agree to some 1e-6
+(4.2e-6 at most here). Without the second f16 term the error is 2^-12 per element, ten times the
+bar. Tokens whose k-th and (k+1)-th router logits lie within 1e-5 of the largest are tie-ambiguous
 and skipped. Routing (indices exactly, weights to 1e-5) is compared with the oracle's
 top_k_routing on the oracle's logits.
 """
