@@ -606,14 +606,14 @@ def chain_check(ctx, M, stack, t_last: int, kernel_opt: int) -> dict:
 
 
 MFMA_FP8_PEAK_TFLOPS = 5000.0  # MI355X dense fp8 (the f8f6f4 MFMA with an fp8 B operand)
-MFMA_INT8_PEAK_TOPS = 5000.0  # MI355X dense int8
+MFMA_F16_PEAK_TFLOPS = 2500.0  # MI355X dense f16
 
 
 def bench_batched(a, ctx, M, W, spec, config, T, K, Wm, cpu_on):
     """One step = one batched forward of T tokens through one layer (router, top-k, grouped
     gate/up + activation, grouped down, combine). C5: 512 tokens through the Zipf-skewed
     GPT-OSS-shape layer; with --batched T on another config: T tokens through its layer 0
-    (Q4_K layers take the grouped int8-MFMA path). Returns the JSON line's object."""
+    (Q4_K layers take the grouped f16-MFMA path). Returns the JSON line's object."""
     dl = W.DeviceLayer(ctx, spec)
     dl.layer.reserve(T)
     H, I = spec.hidden, spec.inter
@@ -645,8 +645,8 @@ def bench_batched(a, ctx, M, W, spec, config, T, K, Wm, cpu_on):
     ctx.sync()
     kern = {}
     for name in ("router_logits", "topk", "group", "split_x", "grouped_gateup", "split_h", "grouped_down",
-                 "split_q4k", "grouped_q4k_gateup", "grouped_q4k_down", "grouped_q4k_shared_gateup",
-                 "grouped_q4k_shared_down", "shared_gate", "combine", "gateup", "down", "shared_gateup"):
+                 "split_q4k", "grouped_q4k_gateup", "grouped_q4k_down", "grouped_shared_gateup",
+                 "grouped_shared_down", "shared_gate", "combine", "gateup", "down", "shared_gateup"):
         n, tot = ctx.profile_read(name)
         if n:
             kern[name] = (n, tot)
@@ -662,14 +662,14 @@ def bench_batched(a, ctx, M, W, spec, config, T, K, Wm, cpu_on):
     if dom in flops:
         ach = flops[dom] / (avg_ms * 1e-3) / 1e12
         q4 = dom.startswith("grouped_q4k")
-        peak = MFMA_INT8_PEAK_TOPS if q4 else MFMA_FP8_PEAK_TFLOPS
+        peak = MFMA_F16_PEAK_TFLOPS if q4 else MFMA_FP8_PEAK_TFLOPS
         tr = measured_traffic(config) if config == 5 and T == W.CONFIG_TOKENS[5] else None
         traffic = int(tr["bytes_per_launch"]) if tr and tr.get("kernel") == dom else None
         roof = {"bound": "mfma", "kernel": dom, "achieved": round(ach, 1), "peak": peak,
-                "unit": "TOP/s" if q4 else "TFLOP/s", "frac": round(ach / peak, 4), "traffic": traffic,
+                "unit": "TFLOP/s", "frac": round(ach / peak, 4), "traffic": traffic,
                 "traffic_source": "profiles/traffic.json (rocprofv3 --pmc)" if traffic else None,
                 "flops_per_launch": flops[dom], "avg_launch_us": round(avg_ms * 1e3, 2),
-                "note": ("GEMM ops of the layer; the 2-term int8 activation split issues 2x this MFMA work"
+                "note": ("GEMM flops of the layer; the 2-term f16 activation split issues 2x this MFMA work"
                          if q4 else "GEMM flops of the layer; the 3-term e4m3 activation split issues 3x this "
                                     "MFMA work")}
     cpu = None
