@@ -208,11 +208,11 @@ struct GQ4Args {
 //   per stage, double buffered, one stage ahead in registers, loaded like the weights, four
 //   lanes per row. In both the 16-byte pieces of a row are spread over the banks (xor).
 //   Nothing in the loop may spill: a reload's wait would drain the prefetched loads (measured:
-//   PG = 1 gate/up 90 us with 36 registers spilled, 50 us with none).
+//   PG = 1 gate/up in 256-row items 90 us with 36 registers spilled, 50 us with none).
 // What bounds it: MFMA and VALU issue, which this chip hardly overlaps (measured on two waves of a
 // SIMD: an MFMA of 16.7 cycles plus four VALU of 2.7 take 26.3), at a clock that falls to 1.7 GHz
-// on long batches: 128 experts of 768 x 2048, 32,768 pairs: gate/up 1.00 -> 0.60 ms and down
-// 0.49 -> 0.32 ms against the int8 MFMA with its scale products on the accumulators per sub-block.
+// on long batches: 128 experts of 768 x 2048, 32,768 pairs: gate/up 1.00 -> 0.54 ms and down
+// 0.49 -> 0.30 ms against the int8 MFMA with its scale products on the accumulators per sub-block.
 // Few pairs: the same unpacking against the weight stream (512 experts of 512 x 2048, 3,840
 // pairs: gate/up 300 -> 191 us, 3.1 TB/s; 128 pairs of 128 experts of 768 x 2048: 78 -> 37 us).
 // 16-row tiles per wave (see the kernel), and the rows of a matrix per work item
